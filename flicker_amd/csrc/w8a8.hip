@@ -68,13 +68,7 @@ __device__ __forceinline__ float wave_max(float v) {
 
 __device__ __forceinline__ float absmax_scale(float amax) { return amax > 0.0f ? amax / kQMax : 1.0f; }
 
-// clamp(rint(v / scale), -127, 127) as an integer.
-__device__ __forceinline__ int quantize(float v, float scale) {
-  const float q = __builtin_rintf(v / scale);
-  return (int)fminf(fmaxf(q, -kQMax), kQMax);
-}
-
-// quantize(v, scale) without a division per element.  r = 1/scale is rounded once per row;
+// clamp(rint(v / scale), -127, 127) as an integer, without a division per element.  r = 1/scale is rounded once per row;
 // p = v * r is then within 3 * 2^-24 |p| < 2^-22 |p| of the correctly rounded quotient q
 // (r, p and q each carry at most half an ulp of relative error).  When p is farther than
 // 2^-21 |p| from a rounding boundary (a half-integer), q lies on the same side and
@@ -120,37 +114,70 @@ __global__ __launch_bounds__(256) void absmax_rows_kernel(const uint16_t* __rest
   if (lane == 0) out[row] = m;
 }
 
-// out[c] = max_r |x[r, c]| (or max with the existing out[c] when accumulating over
-// calibration batches).  A block covers 128 columns: 16 lane groups of 8 columns x 16 row
-// groups, reduced through LDS; each column has exactly one writer.
+// The start of a column maximum: 0, or the running maximum that is accumulated into (a NaN or a
+// negative value there counts as 0, as fmaxf against the first |x| does).
+__global__ __launch_bounds__(256) void absmax_init_kernel(int64_t cols, int accumulate, float* __restrict__ out) {
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (c < cols) out[c] = accumulate ? fmaxf(out[c], 0.0f) : 0.0f;
+}
+
+// Column maxima of one block's 128 columns over rows r, r + 16, ... of [r, r1): 16 lane groups
+// of 8 columns x 16 row groups, kColUnroll rows' loads in flight per thread (a load past r1
+// repeats the thread's first row), reduced through LDS into threads 0-127 (one column each).
+// kScaled: the maximum of |x * s[row]|.
+constexpr int kColUnroll = 8;
+constexpr int kColRows = 16 * kColUnroll;   // rows one pass of a block's loads covers
+
+template <bool kScaled>
+__device__ __forceinline__ float column_absmax(float (&red)[16][129], const uint16_t* __restrict__ x, int64_t stride,
+                                               int64_t r0, int64_t r1, int64_t cols, int64_t c0,
+                                               const float* __restrict__ s) {
+  const int cg = threadIdx.x & 15, rg = threadIdx.x >> 4;
+  float m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (c0 + cg * 8 < cols) {
+    const uint16_t* col = x + c0 + cg * 8;
+    for (int64_t r = r0 + rg; r < r1; r += kColRows) {
+      uint4 v[kColUnroll];
+      float sj[kColUnroll];
+#pragma unroll
+      for (int i = 0; i < kColUnroll; ++i) {
+        const int64_t ri = r + 16 * i < r1 ? r + 16 * i : r;
+        v[i] = *reinterpret_cast<const uint4*>(col + ri * stride);
+        if constexpr (kScaled) sj[i] = s[ri];
+      }
+#pragma unroll
+      for (int i = 0; i < kColUnroll; ++i) {
+        float f[8];
+        unpack_bf16x8(v[i], f);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) m[j] = fmaxf(m[j], fabsf(kScaled ? f[j] * sj[i] : f[j]));
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) red[rg][cg * 8 + j] = m[j];
+  __syncthreads();
+  float v = 0.0f;
+  if (threadIdx.x < 128) {
+#pragma unroll
+    for (int g = 0; g < 16; ++g) v = fmaxf(v, red[g][threadIdx.x]);
+  }
+  return v;
+}
+
+// out[c] = max(out[c], max_r |x[r, c]|), out set by absmax_init_kernel.  HBM-bound: the rows are
+// cut over blockIdx.y so that the pass fills the chip (one block per 128 columns alone was 24
+// blocks at 3072 channels, each a serial walk of the rows).  Block maxima are finite or +inf and
+// never negative, so their int bits order as the floats do and an integer atomic merges them.
+// 4608 x 3072 (28 MB): 6.5 us + 1.6 us to set out, 103 us before.
 __global__ __launch_bounds__(256) void absmax_cols_kernel(const uint16_t* __restrict__ x, int64_t rows,
-                                                          int64_t cols, int64_t stride, int accumulate,
+                                                          int64_t cols, int64_t stride, int64_t rows_per_block,
                                                           float* __restrict__ out) {
   __shared__ float red[16][129];
-  const int cg = threadIdx.x & 15, rg = threadIdx.x >> 4;
-  const int64_t c0 = (int64_t)blockIdx.x * 128 + cg * 8;
-  float m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (c0 < cols) {
-    for (int64_t r = rg; r < rows; r += 16) {
-      float f[8];
-      unpack_bf16x8(*reinterpret_cast<const uint4*>(x + r * stride + c0), f);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) m[i] = fmaxf(m[i], fabsf(f[i]));
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) red[rg][cg * 8 + i] = m[i];
-  __syncthreads();
-  if (threadIdx.x < 128) {
-    const int64_t c = (int64_t)blockIdx.x * 128 + threadIdx.x;
-    if (c < cols) {
-      float v = 0.0f;
-#pragma unroll
-      for (int g = 0; g < 16; ++g) v = fmaxf(v, red[g][threadIdx.x]);
-      if (accumulate) v = fmaxf(v, out[c]);
-      out[c] = v;
-    }
-  }
+  const int64_t c0 = (int64_t)blockIdx.x * 128, r0 = blockIdx.y * rows_per_block;
+  const float v = column_absmax<false>(red, x, stride, r0, min(rows, r0 + rows_per_block), cols, c0, nullptr);
+  const int64_t c = c0 + threadIdx.x;
+  if (threadIdx.x < 128 && c < cols && v > 0.0f) atomicMax(reinterpret_cast<int*>(out) + c, __float_as_int(v));
 }
 
 // s = sqrt(xa) / sqrt(wa) (1 where either maximum is 0), inv_s = 1 / s.
@@ -166,66 +193,76 @@ __global__ void smooth_factors_kernel(const float* __restrict__ xa, const float*
 
 // ---------------------------------------------------------------- quantisation ---------
 
-// Weight (offline): one block per 64 output channels.  Pass 1: column absmax of Wh over all
-// K (8 channel groups x 32 row groups, LDS reduction) -> w_scale.  Pass 2: 64-row k tiles
-// are quantised into an LDS tile [channel][k] and written as 64-byte runs of WqT rows.
+// Weight (offline), three launches.  The first cuts the rows of W over blockIdx.y and writes each
+// cut's column maxima of |Wh| to part (cut, channel); the second takes their maximum -> w_scale;
+// the third quantises.  part is the front of the WqT buffer itself, which the third launch then
+// overwrites: a cut has at least 64 rows, so its 4 bytes per channel fit the K bytes per
+// channel many times over.  HBM-bound; one block per 64 channels walking all the rows twice
+// filled 144 CUs and waited on each row: 3072 x 9216 took 91 us, 31 us now (10.4 + 2.0 + 18.5).
+__global__ __launch_bounds__(256) void weight_absmax_kernel(const uint16_t* __restrict__ w, int64_t w_stride,
+                                                            const float* __restrict__ s, int K, int N,
+                                                            int64_t rows_per_block, float* __restrict__ part) {
+  __shared__ float red[16][129];
+  const int64_t c0 = (int64_t)blockIdx.x * 128, r0 = blockIdx.y * rows_per_block;
+  const float v = column_absmax<true>(red, w, w_stride, r0, min((int64_t)K, r0 + rows_per_block), N, c0, s);
+  const int64_t c = c0 + threadIdx.x;
+  if (threadIdx.x < 128 && c < N) part[(int64_t)blockIdx.y * N + c] = v;
+}
+
+__global__ __launch_bounds__(256) void weight_scale_kernel(const float* __restrict__ part, int cuts, int N,
+                                                           float* __restrict__ w_scale) {
+  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (n >= N) return;
+  float v = 0.0f;
+#pragma unroll 8
+  for (int i = 0; i < cuts; ++i) v = fmaxf(v, part[(int64_t)i * N + n]);
+  w_scale[n] = absmax_scale(v);
+}
+
+// Quantises and transposes one tile of 128 rows (k) x 64 channels.  A thread takes 4 consecutive
+// k of 8 channels, so that four codes leave as one 32-bit LDS write and a WqT row piece as 128
+// contiguous bytes; the 33-word pitch spreads the 64 words of a wave's write over the banks.
 __global__ __launch_bounds__(256) void quantize_weight_kernel(const uint16_t* __restrict__ w, int64_t w_stride,
                                                               const float* __restrict__ s, int K, int N,
                                                               int8_t* __restrict__ wqt,
-                                                              float* __restrict__ w_scale) {
-  __shared__ float red[32][65];
-  __shared__ float scale[64];
-  __shared__ __attribute__((aligned(16))) uint8_t tile[64][80];
+                                                              const float* __restrict__ w_scale) {
+  __shared__ uint32_t tile[64][33];
   const int tid = threadIdx.x;
-  const int cg = tid & 7, rg = tid >> 3;
-  const int n0 = blockIdx.x * 64;
-  const int nc = n0 + cg * 8;
+  const int cg = tid & 7, rq = tid >> 3;
+  const int n0 = blockIdx.x * 64, nc = n0 + cg * 8;
   const bool active = nc < N;
-
-  float m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (active) {
-    for (int j = rg; j < K; j += 32) {
-      const float sj = s[j];
-      float f[8];
-      unpack_bf16x8(*reinterpret_cast<const uint4*>(w + (int64_t)j * w_stride + nc), f);
+  float sc[8], rc[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) m[i] = fmaxf(m[i], fabsf(f[i] * sj));
-    }
-  }
+  for (int j = 0; j < 8; ++j) sc[j] = active ? w_scale[nc + j] : 1.0f;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) red[rg][cg * 8 + i] = m[i];
-  __syncthreads();
-  if (tid < 64) {
-    float v = 0.0f;
-#pragma unroll 8
-    for (int g = 0; g < 32; ++g) v = fmaxf(v, red[g][tid]);
-    const float sc = absmax_scale(v);
-    scale[tid] = sc;
-    if (n0 + tid < N) w_scale[n0 + tid] = sc;
-  }
-  __syncthreads();
-
-  float sc[8];
+  for (int j = 0; j < 8; ++j) rc[j] = 1.0f / sc[j];
+  // One tile, but for a K past the grid's 65535 tiles.
+  for (int64_t k0 = (int64_t)blockIdx.y * 128; k0 < K; k0 += (int64_t)gridDim.y * 128) {
+    const int64_t kr = k0 + rq * 4;
+    if (active && kr < K) {
+      uint4 raw[4];
+      float sj[4], f[4][8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) sc[i] = scale[cg * 8 + i];
-  for (int k0 = 0; k0 < K; k0 += 64) {
+      for (int i = 0; i < 4; ++i) {
+        raw[i] = *reinterpret_cast<const uint4*>(w + (kr + i) * w_stride + nc);
+        sj[i] = s[kr + i];
+      }
 #pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      const int r = rg + it * 32;
-      const int j = k0 + r;
-      if (active) {
-        const float sj = s[j];
-        float f[8];
-        unpack_bf16x8(*reinterpret_cast<const uint4*>(w + (int64_t)j * w_stride + nc), f);
+      for (int i = 0; i < 4; ++i) unpack_bf16x8(raw[i], f[i]);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) tile[cg * 8 + i][r] = (uint8_t)quantize(f[i] * sj, sc[i]);
+      for (int j = 0; j < 8; ++j) {
+        auto qz = [&](int i) { return quantize_recip(f[i][j] * sj[i], sc[j], rc[j]); };
+        tile[cg * 8 + j][rq] = pack_i8x4(qz(0), qz(1), qz(2), qz(3));
       }
     }
     __syncthreads();
-    const int n = tid >> 2, ch = tid & 3;
-    if (n0 + n < N)
-      *reinterpret_cast<uint4*>(wqt + (int64_t)(n0 + n) * K + k0 + ch * 16) =
-          *reinterpret_cast<const uint4*>(&tile[n][ch * 16]);
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const int n = (tid >> 3) + it * 32, ch = tid & 7;
+      if (n0 + n < N && k0 + ch * 16 < K)
+        *reinterpret_cast<uint4*>(wqt + (int64_t)(n0 + n) * K + k0 + ch * 16) =
+            uint4{tile[n][ch * 4], tile[n][ch * 4 + 1], tile[n][ch * 4 + 2], tile[n][ch * 4 + 3]};
+    }
     __syncthreads();
   }
 }
@@ -786,6 +823,14 @@ __global__ __launch_bounds__(kGThreads, 2) void w8a8_gemm_kernel(const GemmGroup
 
 inline hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 
+// Rows per block of a column-maximum launch with `blocks` blocks of 128 columns: one pass of
+// kColRows rows while the grid stays under ~8 blocks per CU, more passes beyond that.
+int64_t column_rows(int64_t rows, int64_t blocks) {
+  const int64_t cuts = std::max<int64_t>(1, 8 * kCUs / blocks);
+  const int64_t per = (rows + cuts - 1) / cuts;
+  return (per + kColRows - 1) / kColRows * kColRows;
+}
+
 }  // namespace
 
 extern "C" int flk_absmax_rows(const void* x, int64_t rows, int64_t cols, int64_t row_stride, float* out,
@@ -810,8 +855,13 @@ extern "C" int flk_absmax_cols(const void* x, int64_t rows, int64_t cols, int64_
     return FLK_E_ALIGN;
   const int64_t blocks = (cols + 127) / 128;
   if (blocks > INT32_MAX) return FLK_E_INVALID;
-  hipLaunchKernelGGL(absmax_cols_kernel, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream),
-                     static_cast<const uint16_t*>(x), rows, cols, row_stride, accumulate, out);
+  hipLaunchKernelGGL(absmax_init_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, as_stream(stream), cols,
+                     accumulate, out);
+  if (rows > 0) {
+    const int64_t per = column_rows(rows, blocks);
+    hipLaunchKernelGGL(absmax_cols_kernel, dim3((unsigned)blocks, (unsigned)((rows + per - 1) / per)), dim3(256), 0,
+                       as_stream(stream), static_cast<const uint16_t*>(x), rows, cols, row_stride, per, out);
+  }
   return flk_launch_status();
 }
 
@@ -837,8 +887,19 @@ extern "C" int flk_quantize_weight(const void* w, int64_t w_row_stride, const fl
   if (!flk_host_aligned(w, 16) || !flk_host_aligned(wq_t, 16) || !flk_host_aligned(s, 4) ||
       !flk_host_aligned(w_scale, 4))
     return FLK_E_ALIGN;
-  hipLaunchKernelGGL(quantize_weight_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, as_stream(stream),
-                     static_cast<const uint16_t*>(w), w_row_stride, s, k, n, wq_t, w_scale);
+  const int64_t col_blocks = ((int64_t)n + 127) / 128;
+  const int64_t per = column_rows(k, col_blocks);
+  const int cuts = (int)(((int64_t)k + per - 1) / per);
+  const int64_t k_tiles = std::min<int64_t>(((int64_t)k + 127) / 128, 65535);   // grid y
+  const hipStream_t hs = as_stream(stream);
+  const uint16_t* wp = static_cast<const uint16_t*>(w);
+  float* part = reinterpret_cast<float*>(wq_t);
+  hipLaunchKernelGGL(weight_absmax_kernel, dim3((unsigned)col_blocks, (unsigned)cuts), dim3(256), 0, hs, wp,
+                     w_row_stride, s, k, n, per, part);
+  hipLaunchKernelGGL(weight_scale_kernel, dim3((unsigned)(((int64_t)n + 255) / 256)), dim3(256), 0, hs, part, cuts, n,
+                     w_scale);
+  hipLaunchKernelGGL(quantize_weight_kernel, dim3((unsigned)((n + 63) / 64), (unsigned)k_tiles), dim3(256), 0, hs, wp,
+                     w_row_stride, s, k, n, wq_t, w_scale);
   return flk_launch_status();
 }
 

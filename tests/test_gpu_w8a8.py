@@ -108,6 +108,37 @@ def test_quantize_weight_full_size_bit_exact(device):
     np.testing.assert_array_equal(host(wq_t), wq_want.T)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 8), (15, 136), (129, 128), (2 * 128 * 16 + 17, 264), (40000, 8)])
+def test_absmax_cols_row_cuts(device, rows, cols):
+    """Row counts around the 128 rows of a block's pass and past one cut per block, into a fresh
+    output, into a running maximum and into one that holds a NaN and a negative value."""
+    g = torch.Generator().manual_seed(rows + cols)
+    x = torch.randn((rows, cols), generator=g).to(torch.bfloat16)
+    x[rows // 2, cols // 2] = float("nan")     # a NaN element is no maximum
+    x[rows - 1, 0] = -float("inf")
+    want = np.nan_to_num(np.abs(x.float().numpy()), nan=0.0, posinf=np.inf).max(0)
+    xd = x.to(device)
+    np.testing.assert_array_equal(host(w8a8.absmax_cols(xd)), want)
+    start = torch.full((cols,), 0.75)
+    start[1], start[2] = float("nan"), -4.0
+    run = w8a8.absmax_cols(xd, out=start.to(device))
+    np.testing.assert_array_equal(host(run), np.maximum(want, np.nan_to_num(start.numpy().clip(min=0.0))))
+
+
+@pytest.mark.parametrize("k,n", [(64, 8), (192, 72), (128, 264), (4096 + 64, 136)])
+def test_quantize_weight_tile_edges(device, k, n):
+    """k of half a 128-row tile and of several cuts, n off the 64- and 128-channel blocks; every
+    byte of WqT is written (the launch uses its front as scratch)."""
+    g = torch.Generator().manual_seed(k + n)
+    w = (0.02 * torch.randn((k, n), generator=g)).to(torch.bfloat16)
+    w[:, n - 1] = 0.0                           # a zero channel: scale 1, codes 0
+    s = (0.5 + torch.rand(k, generator=g)).numpy()
+    wq_want, ws_want = Q.quantize_weight(w.float().numpy(), s)
+    wq_t, ws = w8a8.quantize_weight(w.to(device), torch.from_numpy(s).to(device))
+    np.testing.assert_array_equal(host(ws), ws_want)
+    np.testing.assert_array_equal(host(wq_t), wq_want.T)
+
+
 @pytest.mark.parametrize("strided", [False, True])
 def test_quantize_act_bit_exact(device, strided):
     p = workloads.PROJECTIONS["qkv_1024"]
