@@ -43,6 +43,9 @@
 // partial last round has up to 4/3 as many blocks with 3/4 of the work each (measured 1-5%
 // faster for the plain GEMM, 3-6% with the qk_prep epilogue).
 //
+// A launch of few tiles (a short text stream, a small image) takes tiles of 128 channels x 64 or
+// 128 tokens instead, two waves per 128 x 32 position (gemm_tile_split; launch_group's rule).
+//
 // A launch takes up to two problems (GemmGroup; the activation quantiser likewise takes a
 // QuantGroup): a double block's text and image projections share one grid, so the small
 // text projection runs on the CUs the image projection leaves idle in its last round.
@@ -491,6 +494,134 @@ struct GemmGroup {
   int rounds;   // rounds order (w8a8_gemm_kernel)
 };
 
+// The epilogue of a wave's 128 channels from nw x 16 kMF tokens from mw, of which tokens below
+// m_limit are stored; out_lds holds 16 kMF rows of 256 bytes.  kAcc, kQk, kScaleF32 as for
+// w8a8_gemm_kernel.
+template <bool kAcc, bool kQk, bool kScaleF32, int kMF>
+__device__ __forceinline__ void gemm_epilogue(uint8_t* out_lds, const GemmProblem& P, const i32x4 (&acc)[kGNF][kMF],
+                                              int mw, int nw, int m_limit) {
+  constexpr int kWaveM = 16 * kMF;
+  const int lane = threadIdx.x & 63;
+  const int l16 = lane & 15, h4 = lane >> 4;
+  const float* __restrict__ a_scale = P.a_scale;
+  const float* __restrict__ w_scale = P.w_scale;
+  uint16_t* __restrict__ y = P.y;
+  const int64_t y_stride = P.y_stride;
+  int32_t* __restrict__ acc_out = P.acc_out;
+  const int M = P.M, N = P.N;
+  const QkEpilogue& qe = P.qe;
+  if constexpr (kAcc) {
+    // Exact int32 products, straight from the accumulators: the lane owns token l16 and
+    // channels 4 * (lane / 16) .. +3 of each 16 x 16 fragment.
+#pragma unroll
+    for (int nf = 0; nf < kGNF; ++nf) {
+      const int n = nw + nf * 16 + h4 * 4;
+#pragma unroll
+      for (int mf = 0; mf < kMF; ++mf) {
+        const int m = mw + mf * 16 + l16;
+        if (n < N && m < m_limit) *reinterpret_cast<i32x4*>(acc_out + (int64_t)m * N + n) = acc[nf][mf];
+      }
+    }
+  }
+
+  // Epilogue.  The lane owns token m = mf*16 + l16 and channels n = nf*16 + 4 h4 .. +3 of the
+  // wave's 128 x 64 sub-tile.  Rescaled bf16 values go to this wave's 16 KiB of the (now
+  // idle) LDS as [m][n] rows of 256 B whose 16-byte chunks are XOR-swizzled by m & 15; then
+  // the wave reads back 4 rows per instruction (16 lanes x 16 B per row) and writes each
+  // row's 256 contiguous bytes with 16-byte nontemporal stores (Y is streamed out: 1-2%
+  // faster, and a qk_prep pass reading Y next measured no slower).
+  float am[kMF];
+#pragma unroll
+  for (int mf = 0; mf < kMF; ++mf) am[mf] = a_scale[min(mw + mf * 16 + l16, M - 1)];
+  __syncthreads();   // every wave is done reading the operand stages
+#pragma unroll
+  for (int nf = 0; nf < kGNF; ++nf) {
+    // w_o of the lane's 4 channels (clamped at the edge; clamped values are never stored)
+    const f32x4 w4 = *reinterpret_cast<const f32x4*>(w_scale + min(nw + nf * 16 + h4 * 4, N - 4));
+#pragma unroll
+    for (int mf = 0; mf < kMF; ++mf) {
+      const int ml = mf * 16 + l16;
+      const float y0 = ((float)acc[nf][mf][0] * am[mf]) * w4.x;
+      const float y1 = ((float)acc[nf][mf][1] * am[mf]) * w4.y;
+      const float y2 = ((float)acc[nf][mf][2] * am[mf]) * w4.z;
+      const float y3 = ((float)acc[nf][mf][3] * am[mf]) * w4.w;
+      uint2 packed;
+      packed.x = flk::pack_bf16x2(y0, y1);
+      packed.y = flk::pack_bf16x2(y2, y3);
+      const int chunk = (nf * 2 + (h4 >> 1)) ^ (ml & 15);
+      *reinterpret_cast<uint2*>(out_lds + ml * 256 + chunk * 16 + (h4 & 1) * 8) = packed;
+    }
+  }
+  // Each wave reads back only what it wrote itself: its LDS writes complete in order before
+  // its reads (the compiler waits on lgkmcnt), so no barrier is needed here.
+  constexpr int kReads = kWaveM / 4;
+  const int n_lane = nw + (lane & 15) * 8;
+  if constexpr (kQk) {
+    // The wave's 128 channels are one head of the q|k|v thirds (N = 3 H 128, tiles 128-aligned);
+    // each 16-lane row of a read-back is one token's finished bf16 head row -- the input of
+    // qk_prep, rounded exactly as the unfused path stores it in Y.
+    const int head_g = nw / flk::kQkHeadDim;
+    if (nw >= N) return;
+    const int sec = head_g / qe.heads, h = head_g - sec * qe.heads;
+    float sc[8];
+    if (sec < 2) flk::load_scale8<kScaleF32>(sec == 0 ? qe.q_scale : qe.k_scale, l16, sc);
+    uint16_t* const out = qe.out[sec];
+    // Row m = b * length + t.  One division for the lane's first row; each read-back moves 4
+    // rows on, which wraps into the next batch entry at most once when length >= 4 (shorter
+    // sequences divide per row).  A division per row measured 2.4% of the fused kernel.
+    const int len = qe.length;
+    const bool short_seq = len < 4;
+    const int m_first = mw + (lane >> 4);
+    int b = m_first / len, t = m_first - b * len;
+#pragma unroll 4
+    for (int it = 0; it < kReads; ++it) {
+      const int ml = it * 4 + (lane >> 4);
+      const int m = mw + ml;
+      if (it > 0) {
+        if (short_seq) {
+          b = m / len;
+          t = m - b * len;
+        } else {
+          t += 4;
+          if (t >= len) {
+            t -= len;
+            ++b;
+          }
+        }
+      }
+      const uint4 v = *reinterpret_cast<const uint4*>(out_lds + ml * 256 + ((l16 ^ (ml & 15)) * 16));
+      if (m >= m_limit) continue;   // uniform over the 16-lane row, so the DPP rows stay whole
+      uint4 r = v;
+      if (sec < 2) {
+        float c[8], s[8];
+        flk::load_table8(qe.cos + (int64_t)t * qe.table_stride, l16, c);
+        flk::load_table8(qe.sin + (int64_t)t * qe.table_stride, l16, s);
+        r = sec == 0 ? flk::norm_rotate<kScaleF32, true>(v, sc, c, s, qe.q_gain)
+                     : flk::norm_rotate<kScaleF32, false>(v, sc, c, s, 1.0f);
+      }
+      const int64_t o = (((int64_t)b * qe.heads + h) * qe.out_length + qe.out_offset + t) * flk::kQkHeadDim + l16 * 8;
+      *reinterpret_cast<uint4*>(out + o) = r;
+    }
+    return;
+  }
+  const bool wide = (y_stride & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;   // 16-byte rows
+#pragma unroll 8
+  for (int it = 0; it < kReads; ++it) {
+    const int ml = it * 4 + (lane >> 4);
+    const uint4 v = *reinterpret_cast<const uint4*>(out_lds + ml * 256 + (((lane & 15) ^ (ml & 15)) * 16));
+    const int m = mw + ml;
+    if (m < m_limit && n_lane < N) {
+      uint16_t* dst = y + (int64_t)m * y_stride + n_lane;
+      if (wide && n_lane + 8 <= N) {
+        __builtin_nontemporal_store(u32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4*>(dst));
+      } else {
+        *reinterpret_cast<uint2*>(dst) = uint2{v.x, v.y};
+        if (n_lane + 8 <= N) *reinterpret_cast<uint2*>(dst + 4) = uint2{v.z, v.w};
+      }
+    }
+  }
+}
+
 // One output tile: channels n0 .. n0 + 255 and tokens m0 .. m0 + 64 kMF - 1 (kMF = 4: 256
 // tokens; 3: 192), of which tokens below m_limit are stored.  Each of the 2 (channels) x 4
 // (tokens) waves holds 128 channels x 16 kMF tokens.  kAcc, kQk, kScaleF32 as for
@@ -503,13 +634,7 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const GemmProblem& P, i
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int8_t* __restrict__ xq = P.xq;
   const int8_t* __restrict__ wqt = P.wqt;
-  const float* __restrict__ a_scale = P.a_scale;
-  const float* __restrict__ w_scale = P.w_scale;
-  uint16_t* __restrict__ y = P.y;
-  const int64_t y_stride = P.y_stride;
-  int32_t* __restrict__ acc_out = P.acc_out;
   const int M = P.M, K = P.K, N = P.N;
-  const QkEpilogue& qe = P.qe;
 
   // Copy sources: this wave fills rows wave*32 .. +31 of WqT and wave*8kMF .. +8kMF-1 of Xq,
   // 8 rows (64 lanes x 16 B) per instruction; lane i lands at row i/8, slot i%8, and fetches
@@ -621,118 +746,119 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const GemmProblem& P, i
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  if constexpr (kAcc) {
-    // Exact int32 products, straight from the accumulators: the lane owns token l16 and
-    // channels 4 * (lane / 16) .. +3 of each 16 x 16 fragment.
+  gemm_epilogue<kAcc, kQk, kScaleF32, kMF>(smem + wave * (kWaveM * 256), P, acc, m0 + wm * kWaveM,
+                                           n0 + wn * kGWaveN, m_limit);
+}
+
+// The same product for launches whose 256 x 256 tiles leave most CUs idle: tiles of 128 channels x
+// 32 kWM tokens, taken by 2 kWM waves.  A 128 x 32 position is held by two waves that take the two
+// 64-byte halves of every 128-byte k stage; their int32 sums (exact in any order) are exchanged
+// through LDS at the end, each wave finishing 16 of the 32 tokens.  Few blocks run a serial chain
+// of stages, so what bounds it is a stage's latency: two waves per SIMD on one position halve the
+// chain's MFMAs per wave (four waves with whole stages: 27 us against 22.6 at 512 tokens).
+template <bool kAcc, bool kQk, bool kScaleF32, int kWM, int kBuffers>
+__device__ __forceinline__ void gemm_tile_split(uint8_t* smem, const GemmProblem& P, int m0, int n0, int m_limit) {
+  constexpr int kMF = 2, kWaveM = 16 * kMF, kWaves = 2 * kWM, kTM = kWM * kWaveM;
+  constexpr int kABytes = kGWaveN * kGK, kStage = kABytes + kTM * kGK;
+  constexpr int kAC = kGWaveN / 8 / kWaves, kBC = kTM / 8 / kWaves;   // copies per wave and stage (8 rows each)
+  static_assert(kGWaveN % (8 * kWaves) == 0 && kTM % (8 * kWaves) == 0, "whole copies per wave");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int M = P.M, K = P.K, N = P.N;
+  const int8_t* abase = P.wqt + (int64_t)n0 * K;
+  const int8_t* bbase = P.xq + (int64_t)m0 * K;
+  uint32_t aoff[kAC], boff[kBC];
+#pragma unroll
+  for (int i = 0; i < kAC; ++i) {
+    const int row = (wave * kAC + i) * 8 + (lane >> 3);
+    aoff[i] = (uint32_t)min(row, N - 1 - n0) * (uint32_t)K + (uint32_t)(((lane & 7) ^ gswz(row)) * 16);
+  }
+#pragma unroll
+  for (int i = 0; i < kBC; ++i) {
+    const int row = (wave * kBC + i) * 8 + (lane >> 3);
+    boff[i] = (uint32_t)min(row, M - 1 - m0) * (uint32_t)K + (uint32_t)(((lane & 7) ^ gswz(row)) * 16);
+  }
+  const int kg = wave / kWM, wm = wave % kWM;   // half of the k stages, 32-token position
+  const int l16 = lane & 15, h4 = lane >> 4;
+  const int hperm = ((h4 & 1) << 1) | (h4 >> 1);
+  const int off = l16 * kGK + (((4 * kg + hperm) ^ gswz(l16)) * 16);
+  const int b_off = off + kABytes + wm * kWaveM * kGK;
+
+  i32x4 acc[kGNF][kMF];
+#pragma unroll
+  for (int a = 0; a < kGNF; ++a)
+#pragma unroll
+    for (int b = 0; b < kMF; ++b) acc[a][b] = i32x4{};
+
+  const int KT = K / kGK;
+  auto copy_stage = [&](int kt, uint8_t* dst) {
+    const int k_off = min(kt, KT - 1) * kGK;
+#pragma unroll
+    for (int i = 0; i < kAC; ++i) flk::dma16_at(abase + k_off, aoff[i], dst + (wave * kAC + i) * 8 * kGK);
+#pragma unroll
+    for (int i = 0; i < kBC; ++i) flk::dma16_at(bbase + k_off, boff[i], dst + kABytes + (wave * kBC + i) * 8 * kGK);
+  };
+#pragma unroll
+  for (int i = 0; i < kBuffers; ++i) copy_stage(i, smem + i * kStage);
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"((kBuffers - 1) * (kAC + kBC)) : "memory");
+  __syncthreads();
+  auto afrag = [&](const uint8_t* st, int nf) { return *reinterpret_cast<const i32x4*>(st + off + nf * 16 * kGK); };
+  auto bfrag = [&](const uint8_t* st, int mf) { return *reinterpret_cast<const i32x4*>(st + b_off + mf * 16 * kGK); };
+  i32x4 ring[kGRing], b0[kMF], b1[kMF];
+#pragma unroll
+  for (int mf = 0; mf < kMF; ++mf) b0[mf] = bfrag(smem, mf);
+#pragma unroll
+  for (int nf = 0; nf < kGLead; ++nf) ring[nf] = afrag(smem, nf);
+
+  int cb = 0;   // byte offset of stage kt's buffer
+  auto step = [&](int kt, i32x4 (&b)[kMF], i32x4 (&bn)[kMF]) {
+    uint8_t* cs = smem + cb;
+    cb = cb == (kBuffers - 1) * kStage ? 0 : cb + kStage;
+    const uint8_t* ns = smem + cb;
 #pragma unroll
     for (int nf = 0; nf < kGNF; ++nf) {
-      const int n = n0 + wn * kGWaveN + nf * 16 + h4 * 4;
 #pragma unroll
-      for (int mf = 0; mf < kMF; ++mf) {
-        const int m = m0 + wm * kWaveM + mf * 16 + l16;
-        if (n < N && m < m_limit) *reinterpret_cast<i32x4*>(acc_out + (int64_t)m * N + n) = acc[nf][mf];
+      for (int mf = 0; mf < kMF; ++mf)
+        acc[nf][mf] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ring[nf % kGRing], b[mf], acc[nf][mf], 0, 0, 0);
+      const int nl = nf + kGLead;
+      ring[nl % kGRing] = nl < kGNF ? afrag(cs, nl) : afrag(ns, nl - kGNF);
+      if (nf >= kGNF - kGLead) {
+        const int j = nf - (kGNF - kGLead);
+#pragma unroll
+        for (int mf = 0; mf < kMF; ++mf)
+          if (mf * kGLead / kMF == j) bn[mf] = bfrag(ns, mf);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (nf == kGNF - kGLead - 1) {
+        // every wave has read stage kt; stage kt+1 has landed everywhere
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((kBuffers - 2) * (kAC + kBC)) : "memory");
+        copy_stage(kt + kBuffers, cs);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
+  };
+  int kt = 0;
+  for (; kt + 2 <= KT; kt += 2) {
+    step(kt, b0, b1);
+    step(kt + 1, b1, b0);
   }
-
-  // Epilogue.  The lane owns token m = mf*16 + l16 and channels n = nf*16 + 4 h4 .. +3 of the
-  // wave's 128 x 64 sub-tile.  Rescaled bf16 values go to this wave's 16 KiB of the (now
-  // idle) LDS as [m][n] rows of 256 B whose 16-byte chunks are XOR-swizzled by m & 15; then
-  // the wave reads back 4 rows per instruction (16 lanes x 16 B per row) and writes each
-  // row's 256 contiguous bytes with 16-byte nontemporal stores (Y is streamed out: 1-2%
-  // faster, and a qk_prep pass reading Y next measured no slower).
-  float am[kMF];
-#pragma unroll
-  for (int mf = 0; mf < kMF; ++mf) am[mf] = a_scale[min(m0 + wm * kWaveM + mf * 16 + l16, M - 1)];
-  __syncthreads();   // every wave is done reading the operand stages
-  uint8_t* const out_lds = smem + wave * (kWaveM * 256);
+  if (kt < KT) step(kt, b0, b1);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  // Wave kg of a position keeps token fragment kg and gives the other one away.
+  i32x4* const sums = reinterpret_cast<i32x4*>(smem) + lane;
+  constexpr int kSum = kGNF * 64;   // one wave's fragments
+  static_assert(kWaves * kSum * 16 <= kBuffers * kStage, "the exchanged sums fit the idle stages");
+  i32x4 sum[kGNF][1];
 #pragma unroll
   for (int nf = 0; nf < kGNF; ++nf) {
-    // w_o of the lane's 4 channels (clamped at the edge; clamped values are never stored)
-    const f32x4 w4 = *reinterpret_cast<const f32x4*>(w_scale + min(n0 + wn * kGWaveN + nf * 16 + h4 * 4, N - 4));
+    sums[wave * kSum + nf * 64] = kg ? acc[nf][0] : acc[nf][1];
+    sum[nf][0] = kg ? acc[nf][1] : acc[nf][0];
+  }
+  __syncthreads();
 #pragma unroll
-    for (int mf = 0; mf < kMF; ++mf) {
-      const int ml = mf * 16 + l16;
-      const float y0 = ((float)acc[nf][mf][0] * am[mf]) * w4.x;
-      const float y1 = ((float)acc[nf][mf][1] * am[mf]) * w4.y;
-      const float y2 = ((float)acc[nf][mf][2] * am[mf]) * w4.z;
-      const float y3 = ((float)acc[nf][mf][3] * am[mf]) * w4.w;
-      uint2 packed;
-      packed.x = flk::pack_bf16x2(y0, y1);
-      packed.y = flk::pack_bf16x2(y2, y3);
-      const int chunk = (nf * 2 + (h4 >> 1)) ^ (ml & 15);
-      *reinterpret_cast<uint2*>(out_lds + ml * 256 + chunk * 16 + (h4 & 1) * 8) = packed;
-    }
-  }
-  // Each wave reads back only what it wrote itself: its LDS writes complete in order before
-  // its reads (the compiler waits on lgkmcnt), so no barrier is needed here.
-  constexpr int kReads = kWaveM / 4;
-  const int n_lane = n0 + wn * kGWaveN + (lane & 15) * 8;
-  if constexpr (kQk) {
-    // The wave's 128 channels are one head of the q|k|v thirds (N = 3 H 128, tiles 128-aligned);
-    // each 16-lane row of a read-back is one token's finished bf16 head row -- the input of
-    // qk_prep, rounded exactly as the unfused path stores it in Y.
-    const int head_g = (n0 + wn * kGWaveN) / flk::kQkHeadDim;
-    if (n0 + wn * kGWaveN >= N) return;
-    const int sec = head_g / qe.heads, h = head_g - sec * qe.heads;
-    const int l16 = lane & 15;
-    float sc[8];
-    if (sec < 2) flk::load_scale8<kScaleF32>(sec == 0 ? qe.q_scale : qe.k_scale, l16, sc);
-    uint16_t* const out = qe.out[sec];
-    // Row m = b * length + t.  One division for the lane's first row; each read-back moves 4
-    // rows on, which wraps into the next batch entry at most once when length >= 4 (shorter
-    // sequences divide per row).  A division per row measured 2.4% of the fused kernel.
-    const int len = qe.length;
-    const bool short_seq = len < 4;
-    const int m_first = m0 + wm * kWaveM + (lane >> 4);
-    int b = m_first / len, t = m_first - b * len;
-#pragma unroll 4
-    for (int it = 0; it < kReads; ++it) {
-      const int ml = it * 4 + (lane >> 4);
-      const int m = m0 + wm * kWaveM + ml;
-      if (it > 0) {
-        if (short_seq) {
-          b = m / len;
-          t = m - b * len;
-        } else {
-          t += 4;
-          if (t >= len) {
-            t -= len;
-            ++b;
-          }
-        }
-      }
-      const uint4 v = *reinterpret_cast<const uint4*>(out_lds + ml * 256 + ((l16 ^ (ml & 15)) * 16));
-      if (m >= m_limit) continue;   // uniform over the 16-lane row, so the DPP rows stay whole
-      uint4 r = v;
-      if (sec < 2) {
-        float c[8], s[8];
-        flk::load_table8(qe.cos + (int64_t)t * qe.table_stride, l16, c);
-        flk::load_table8(qe.sin + (int64_t)t * qe.table_stride, l16, s);
-        r = sec == 0 ? flk::norm_rotate<kScaleF32, true>(v, sc, c, s, qe.q_gain)
-                     : flk::norm_rotate<kScaleF32, false>(v, sc, c, s, 1.0f);
-      }
-      const int64_t o = (((int64_t)b * qe.heads + h) * qe.out_length + qe.out_offset + t) * flk::kQkHeadDim + l16 * 8;
-      *reinterpret_cast<uint4*>(out + o) = r;
-    }
-    return;
-  }
-  const bool wide = (y_stride & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;   // 16-byte rows
-#pragma unroll 8
-  for (int it = 0; it < kReads; ++it) {
-    const int ml = it * 4 + (lane >> 4);
-    const uint4 v = *reinterpret_cast<const uint4*>(out_lds + ml * 256 + (((lane & 15) ^ (ml & 15)) * 16));
-    const int m = m0 + wm * kWaveM + ml;
-    if (m < m_limit && n_lane < N) {
-      uint16_t* dst = y + (int64_t)m * y_stride + n_lane;
-      if (wide && n_lane + 8 <= N) {
-        __builtin_nontemporal_store(u32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4*>(dst));
-      } else {
-        *reinterpret_cast<uint2*>(dst) = uint2{v.x, v.y};
-        if (n_lane + 8 <= N) *reinterpret_cast<uint2*>(dst + 4) = uint2{v.z, v.w};
-      }
-    }
-  }
+  for (int nf = 0; nf < kGNF; ++nf) sum[nf][0] += sums[((1 - kg) * kWM + wm) * kSum + nf * 64];
+  gemm_epilogue<kAcc, kQk, kScaleF32, 1>(smem + wave * (16 * 256), P, sum, m0 + wm * kWaveM + kg * 16, n0, m_limit);
 }
 
 // Logical tile u of a problem -> its token and channel tiles: kGroup token tiles sweep the
@@ -819,6 +945,21 @@ __global__ __launch_bounds__(kGThreads, 2) void w8a8_gemm_kernel(const GemmGroup
   int mt, nt;
   tile_of(logical_all - (second ? grp.first_blocks : 0), P.tiles_m, P.tiles_n, mt, nt);
   gemm_tile<kAcc, kQk, kScaleF32, 4>(smem, P, mt * kGT, nt * kGT, P.M);
+}
+
+// A launch of few tiles (launch_group): one tile of 128 channels x 32 kWM tokens per block, through
+// kBuffers LDS stages, kPerCU blocks to a CU.
+template <bool kAcc, bool kQk, bool kScaleF32, int kWM, int kBuffers, int kPerCU>
+__global__ __launch_bounds__(kWM * 128, kPerCU * kWM / 2) void w8a8_gemm_split_kernel(const GemmGroup grp) {
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kBuffers * (kGWaveN + 32 * kWM) * kGK];
+  const int xcd = blockIdx.x % kXcds, local = blockIdx.x / kXcds;   // blocks are dealt round-robin over XCDs
+  const int per = gridDim.x / kXcds, extra = gridDim.x % kXcds;
+  const int logical = xcd * per + min(xcd, extra) + local;
+  const bool second = logical >= grp.first_blocks;
+  const GemmProblem& P = second ? grp.p[1] : grp.p[0];   // wave-uniform, read from the kernel arguments
+  int mt, nt;
+  tile_of(logical - (second ? grp.first_blocks : 0), P.tiles_m, P.tiles_n, mt, nt);
+  gemm_tile_split<kAcc, kQk, kScaleF32, kWM, kBuffers>(smem, P, mt * 32 * kWM, nt * kGWaveN, P.M);
 }
 
 inline hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
@@ -1010,7 +1151,7 @@ extern "C" int flk_quantize_act_modulated_pair(
 
 namespace {
 
-int64_t problem_blocks(const GemmProblem& p) { return (int64_t)p.tiles_m * p.tiles_n; }
+int64_t tiles(int size, int edge) { return ((int64_t)size + edge - 1) / edge; }
 
 // Grid of the rounds order of a launch (w8a8_gemm_kernel), or 0 when it is not the choice: it
 // needs a full round of 32 tiles on every XCD, tiles left over, and at most one round of
@@ -1045,19 +1186,54 @@ int64_t gemm_rounds_grid(const GemmGroup& g) {
   return left_max > 0 ? most * kXcds : 0;
 }
 
-// Fills a launch's tile count and order; returns its grid.
-int64_t plan_group(GemmGroup& g, int64_t units) {
+// Fills a launch's tiles of tm tokens x tn channels (of p[0] alone unless both); returns their count.
+int64_t plan_tiles(GemmGroup& g, bool both, int tm, int tn) {
+  for (GemmProblem& p : g.p) {
+    p.tiles_m = (int)tiles(p.M, tm);
+    p.tiles_n = (int)tiles(p.N, tn);
+  }
+  const int64_t first = (int64_t)g.p[0].tiles_m * g.p[0].tiles_n;
+  g.first_blocks = (int)std::min<int64_t>(first, INT32_MAX);
+  const int64_t units = first + (both ? (int64_t)g.p[1].tiles_m * g.p[1].tiles_n : 0);
   g.units = (int)std::min<int64_t>(units, INT32_MAX);
-  const int64_t rounds = units <= INT32_MAX ? gemm_rounds_grid(g) : 0;
-  g.rounds = rounds > 0;
-  return rounds ? rounds : units;
+  return units;
 }
 
+// Launches p[0], and p[1] when both.  A round of 256 x 256 tiles takes ~34 us at K = 3072 however
+// few blocks it has, so a launch takes the smallest of these tiles that fit the chip at once, the
+// shortest chain per CU (us, plain GEMM with 3072 x 9216 weights, 256 x 256 tiles first):
+//   128 x 64, one block per CU             17 tokens: 33.2 -> 10.3    128 tokens: 34.3 -> 11.3
+//   128 x 128, one per CU, four stages    256 tokens: 34.6 -> 15.1    384 tokens: 34.6 -> 15.5
+//   128 x 128, two per CU, two stages     512 tokens: 34.7 -> 22.6    896 tokens: 39.4 -> 29.3
+// Past that 256 x 256 tiles, with half the stage copies per product, are faster: at 1152 tokens
+// (648 tiles of 128 x 128) 41.7 against 46.2, at 4608 129 against 149.
 template <bool kAcc, bool kQk, bool kScaleF32>
-int launch_group(const GemmGroup& g, int64_t blocks, void* stream) {
+int launch_group(GemmGroup g, bool both, void* stream) {
+  if (!both) g.p[1] = g.p[0];
+  const hipStream_t st = as_stream(stream);
+  int64_t blocks = plan_tiles(g, both, 64, kGWaveN);
+  if (blocks <= kCUs) {
+    hipLaunchKernelGGL((w8a8_gemm_split_kernel<kAcc, kQk, kScaleF32, 2, 4, 1>), dim3((unsigned)blocks), dim3(256), 0,
+                       st, g);
+    return flk_launch_status();
+  }
+  blocks = plan_tiles(g, both, 128, kGWaveN);
+  if (blocks <= kCUs) {
+    hipLaunchKernelGGL((w8a8_gemm_split_kernel<kAcc, kQk, kScaleF32, 4, 4, 1>), dim3((unsigned)blocks), dim3(512), 0,
+                       st, g);
+    return flk_launch_status();
+  }
+  if (blocks <= 2 * kCUs) {
+    hipLaunchKernelGGL((w8a8_gemm_split_kernel<kAcc, kQk, kScaleF32, 4, 2, 2>), dim3((unsigned)blocks), dim3(512), 0,
+                       st, g);
+    return flk_launch_status();
+  }
+  blocks = plan_tiles(g, both, kGT, kGT);
+  const int64_t rounds = blocks <= INT32_MAX ? gemm_rounds_grid(g) : 0;
+  g.rounds = rounds > 0;
+  if (rounds) blocks = rounds;
   if (blocks > INT32_MAX) return FLK_E_INVALID;
-  hipLaunchKernelGGL((w8a8_gemm_kernel<kAcc, kQk, kScaleF32>), dim3((unsigned)blocks), dim3(kGThreads), 0,
-                     as_stream(stream), g);
+  hipLaunchKernelGGL((w8a8_gemm_kernel<kAcc, kQk, kScaleF32>), dim3((unsigned)blocks), dim3(kGThreads), 0, st, g);
   return flk_launch_status();
 }
 
@@ -1092,17 +1268,15 @@ int qk_problem(const int8_t* xq, const int8_t* wq_t, const float* a_scale, const
   p.M = (int)m64;
   p.K = k;
   p.N = (int)n;
-  p.tiles_m = (p.M + kGT - 1) / kGT;
-  p.tiles_n = (p.N + kGT - 1) / kGT;
   p.qe = QkEpilogue{cos, sin, table_row_stride, q_scale, k_scale, q_gain, length, num_heads,
                     {static_cast<uint16_t*>(q_out), static_cast<uint16_t*>(k_out), static_cast<uint16_t*>(v_out)},
                     out_length, out_offset};
   return FLK_OK;
 }
 
-int launch_qk(const GemmGroup& g, int64_t blocks, int scale_is_f32, void* stream) {
-  return scale_is_f32 ? launch_group<false, true, true>(g, blocks, stream)
-                      : launch_group<false, true, false>(g, blocks, stream);
+int launch_qk(const GemmGroup& g, bool both, int scale_is_f32, void* stream) {
+  return scale_is_f32 ? launch_group<false, true, true>(g, both, stream)
+                      : launch_group<false, true, false>(g, both, stream);
 }
 
 }  // namespace
@@ -1132,13 +1306,8 @@ extern "C" int flk_w8a8_gemm(const int8_t* xq, const int8_t* wq_t, const float* 
   p.M = m;
   p.K = k;
   p.N = n;
-  p.tiles_m = (m + kGT - 1) / kGT;
-  p.tiles_n = (n + kGT - 1) / kGT;
-  g.p[1] = p;
-  g.first_blocks = (int)std::min<int64_t>(problem_blocks(p), INT32_MAX);
-  const int64_t blocks = plan_group(g, problem_blocks(p));
-  return acc_or_null ? launch_group<true, false, false>(g, blocks, stream)
-                     : launch_group<false, false, false>(g, blocks, stream);
+  return acc_or_null ? launch_group<true, false, false>(g, false, stream)
+                     : launch_group<false, false, false>(g, false, stream);
 }
 
 extern "C" int flk_w8a8_qk_prep(const int8_t* xq, const int8_t* wq_t, const float* a_scale, const float* w_scale,
@@ -1150,10 +1319,7 @@ extern "C" int flk_w8a8_qk_prep(const int8_t* xq, const int8_t* wq_t, const floa
   const int st = qk_problem(xq, wq_t, a_scale, w_scale, k, cos, sin, table_row_stride, q_scale, k_scale, q_gain,
                             batch, length, num_heads, head_dim, q_out, k_out, v_out, out_length, out_offset, g.p[0]);
   if (st != FLK_OK) return st == kNoWork ? FLK_OK : st;
-  g.p[1] = g.p[0];
-  g.first_blocks = (int)std::min<int64_t>(problem_blocks(g.p[0]), INT32_MAX);
-  const int64_t blocks = plan_group(g, problem_blocks(g.p[0]));
-  return launch_qk(g, blocks, scale_is_f32, stream);
+  return launch_qk(g, false, scale_is_f32, stream);
 }
 
 extern "C" int flk_w8a8_qk_prep_pair(
@@ -1175,10 +1341,5 @@ extern "C" int flk_w8a8_qk_prep_pair(
   if (st0 == kNoWork && st1 == kNoWork) return FLK_OK;
   // An empty problem gives its place to the other one, which then takes every block.
   if (st0 == kNoWork) g.p[0] = g.p[1];
-  if (st1 == kNoWork) g.p[1] = g.p[0];
-  const bool both = st0 == FLK_OK && st1 == FLK_OK;
-  const int64_t b0 = problem_blocks(g.p[0]);
-  g.first_blocks = (int)std::min<int64_t>(b0, INT32_MAX);
-  const int64_t blocks = plan_group(g, both ? b0 + problem_blocks(g.p[1]) : b0);
-  return launch_qk(g, blocks, scale_is_f32, stream);
+  return launch_qk(g, st0 == FLK_OK && st1 == FLK_OK, scale_is_f32, stream);
 }

@@ -220,6 +220,26 @@ def test_gemm_rounds_order_bit_exact(device, m, n):
     assert_bits_equal(y, Q.rescale(acc_want, a, ws), f"y {m}x{k}x{n}")
 
 
+@pytest.mark.parametrize("m,k,n", [(17, 3072, 9216), (192, 384, 9216), (193, 128, 9216), (383, 640, 9212),
+                                   (385, 384, 9216), (895, 256, 9216), (897, 128, 9216), (2048, 384, 4096),
+                                   (2049, 256, 4096)])
+def test_gemm_few_tiles_bit_exact(device, m, k, n):
+    """Both sides of each line between the tile sizes of small launches: 256 tiles of 128 channels
+    x 64 tokens, 256 and 512 of 128 x 128; odd stage counts, fewer stages than LDS buffers, ragged
+    edges.  Integer sums: every product and output bit for bit."""
+    rng = np.random.default_rng(m + k + n)
+    xq = rng.integers(-127, 128, (m, k), dtype=np.int8)
+    wq = rng.integers(-127, 128, (k, n), dtype=np.int8)
+    a = (rng.random(m, dtype=np.float32) * 0.05 + 1e-3).astype(np.float32)
+    ws = (rng.random(n, dtype=np.float32) * 0.002 + 1e-5).astype(np.float32)
+    acc = torch.empty((m, n), dtype=torch.int32, device=device)
+    y = w8a8.gemm(torch.from_numpy(xq).to(device), torch.from_numpy(a).to(device),
+                  torch.from_numpy(np.ascontiguousarray(wq.T)).to(device), torch.from_numpy(ws).to(device), acc=acc)
+    acc_want = Q.int_gemm(xq, wq)
+    np.testing.assert_array_equal(host(acc), acc_want)
+    assert_bits_equal(y, Q.rescale(acc_want, a, ws), f"y {m}x{k}x{n}")
+
+
 def test_gemm_random_shapes_bit_exact(device):
     """Seeded random projections around one round of tiles (some take the rounds order, some
     the plain order, ragged edges in both dimensions): every int32 product and bf16 output
@@ -437,6 +457,7 @@ def test_modulated_projection_qk_prep(device):
     (1, 512, 4096, 24, 3072, torch.bfloat16, False),   # a Klein double block: 512 text + 64x64 image tokens
     (2, 70, 300, 2, 256, torch.float32, True),          # ragged streams, f32 scales, modulated inputs
     (1, 0, 130, 2, 128, torch.bfloat16, False),         # an empty text stream
+    (1, 512, 256, 24, 384, torch.bfloat16, True),       # 128-token tiles of both streams, two per CU
 ])
 def test_fused_projection_pair_equals_two_calls(device, batch, len0, len1, heads, k, scale_dtype, modulated):
     """flk_w8a8_qk_prep_pair (both streams of a double block in one launch) writes exactly what
