@@ -270,8 +270,8 @@ __global__ __launch_bounds__(256) void quantize_weight_kernel(const uint16_t* __
   }
 }
 
-// Activation (per forward): one wave per token row, the row held in registers
-// (kChunks x 8 elements per lane), absmax reduced across the wave.
+// Activation (per forward): kRowWaves waves per token row, the row held in registers
+// (kChunks x 8 elements per lane), its sums and its absmax reduced across the waves.
 //
 // kModulate: the row is first the block input x and becomes the projection input
 //   X = bf16(bf16((bf16(1 + scale) * bf16(layer_norm(x)))) + shift)      (modules.py:38-40)
@@ -280,10 +280,82 @@ __global__ __launch_bounds__(256) void quantize_weight_kernel(const uint16_t* __
 // sum of the row exact, so the mean does not depend on the summation order), every other
 // step one f32 operation.  scale / shift are the modulation rows of the token's batch entry;
 // X is optionally stored (bf16) for other consumers of the modulated input.
-__device__ __forceinline__ double wave_sum(double v) {
+//
+// What bounds it is VALU work and the latency of the chain load -> sum -> sum -> absmax -> codes,
+// not memory: every load is issued before the first reduction, reductions cross lanes by DPP,
+// and the codes take five instructions an element (Codes below).
+template <int kCtrl>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xF, 0xF, false));
+}
+
+template <int kCtrl>
+__device__ __forceinline__ double dpp_move(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, kCtrl, 0xF, 0xF, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), kCtrl, 0xF, 0xF, false);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+// op over the 64 lanes of a wave: the 16-lane rows by DPP, then the rows by lane shuffles.
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce(T v, Op op) {
+  v = op(v, dpp_move<0xB1>(v));    // quad_perm 1,0,3,2
+  v = op(v, dpp_move<0x4E>(v));    // quad_perm 2,3,0,1
+  v = op(v, dpp_move<0x141>(v));   // row_half_mirror
+  v = op(v, dpp_move<0x140>(v));   // row_mirror
+  v = op(v, __shfl_xor(v, 16));
+  return op(v, __shfl_xor(v, 32));
+}
+
+// ... and over the kRowWaves waves of each of kRows rows, through LDS; every thread of the block
+// calls it.
+template <int kRowWaves, int kRows, typename T, typename Op>
+__device__ __forceinline__ void row_reduce(T (&v)[kRows], T (&slot)[4][kRows], Op op) {
 #pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
-  return v;
+  for (int r = 0; r < kRows; ++r) v[r] = wave_reduce(v[r], op);
+  if constexpr (kRowWaves > 1) {
+    const int wave = threadIdx.x >> 6, first = wave / kRowWaves * kRowWaves;
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) slot[wave][r] = v[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      v[r] = slot[first][r];
+#pragma unroll
+      for (int i = 1; i < kRowWaves; ++i) v[r] = op(v[r], slot[first + i][r]);
+    }
+  }
+}
+
+// The codes clamp(rint(v / a), -127, 127) of 8 elements without a division each.  r = 1 / a is
+// rounded once per row, so v * r is within 2^-23 |q| < 1.6e-5 of the correctly rounded quotient q
+// (|q| <= 127.0001: a is the row's absmax / 127).  Adding 1.5 * 2^23 rounds the exact product to
+// its integer t, whose two's complement is then the sum's low byte; when the product is within
+// 0.5 - 2^-15 of t, q rounds to t too.  Otherwise -- near a tie, or not finite -- the lane divides.
+__device__ __forceinline__ uint2 quantize8(const float (&v)[8], float a, float r) {
+  constexpr float kRound = 12582912.0f;
+  uint32_t u[8];
+  bool near = false;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float sum = __builtin_fmaf(v[i], r, kRound);
+    const float off = __builtin_fmaf(v[i], r, -(sum - kRound));
+    near |= !(fabsf(off) < 0.5f - 0x1p-15f);
+    u[i] = __float_as_uint(sum);
+  }
+  if (near) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) u[i] = (uint32_t)(int)fminf(fmaxf(__builtin_rintf(v[i] / a), -kQMax), kQMax);
+  }
+  // bytes 0 of four words: perm selects from (second argument: bytes 0-3, first: 4-7), 0x0c = 0
+  auto pack = [&](int i) {
+    const uint32_t lo = __builtin_amdgcn_perm(u[i + 1], u[i], 0x0c0c0400u);
+    const uint32_t hi = __builtin_amdgcn_perm(u[i + 3], u[i + 2], 0x04000c0cu);
+    return lo | hi;
+  };
+  return uint2{pack(0), pack(4)};
 }
 
 // One activation of a quantisation launch (rows of M tokens, all of width K).
@@ -303,118 +375,164 @@ struct QuantProblem {
 };
 
 // Up to two activations in one launch (a double block's text and image streams): blocks
-// [0, first_blocks) take p[0], the rest p[1]; four rows per block.
+// [0, first_blocks) take p[0], the rest p[1]; 4 / kRowWaves rows per block.
 struct QuantGroup {
   QuantProblem p[2];
   int first_blocks;
   int K;
 };
 
-template <int kChunks, bool kModulate>
+// kRows rows per wave (consecutive, of one batch entry or two): their loads are in flight together
+// and, in one batch entry, they share the modulation.  kFull: the lanes' chunks end with the row.
+template <int kRowWaves, int kChunks, bool kFull, int kRows, bool kModulate>
 __global__ __launch_bounds__(256) void quantize_act_kernel(const QuantGroup grp) {
+  __shared__ double sums[4][kRows], squares[4][kRows];
+  __shared__ float maxima[4][kRows];
   const bool second = (int)blockIdx.x >= grp.first_blocks;
   const QuantProblem& P = second ? grp.p[1] : grp.p[0];   // wave-uniform, read from the kernel arguments
-  const uint16_t* __restrict__ x = P.x;
-  const int64_t x_stride = P.x_stride;
-  const float* __restrict__ inv_s = P.inv_s;
   const int M = P.M, K = grp.K;
-  int8_t* __restrict__ xq = P.xq;
-  float* __restrict__ a_scale = P.a_scale;
-  const uint16_t* __restrict__ shift = P.shift;
-  const uint16_t* __restrict__ scale = P.scale;
-  const int64_t mod_stride = P.mod_stride;
-  const int tokens_per_batch = P.tokens_per_batch;
-  uint16_t* __restrict__ x_mod = P.x_mod;
-  const int64_t x_mod_stride = P.x_mod_stride;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int row = ((int)blockIdx.x - (second ? grp.first_blocks : 0)) * 4 + wave;
-  if (row >= M) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int block = (int)blockIdx.x - (second ? grp.first_blocks : 0);
+  const int64_t row0 = ((int64_t)block * (4 / kRowWaves) + wave / kRowWaves) * kRows;
   const int nch = K >> 3;
-  const uint16_t* src = x + (int64_t)row * x_stride;
-  uint4 raw[kChunks];
+  const int first = wave % kRowWaves * 64 + lane;   // the lane's chunks: first, first + 64 kRowWaves, ...
+  auto chunk = [&](int c) { return first + c * 64 * kRowWaves; };
+  auto valid = [&](int c) { return kFull || chunk(c) < nch; };
+  int row[kRows];   // rows past the end repeat the last one and store nothing
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) row[r] = (int)min(row0 + r, (int64_t)M - 1);
+
+  // Every load unconditional (a chunk past the row's end re-reads chunk 0 and counts as zeros).
+  uint4 raw[kRows][kChunks];
+#pragma unroll
+  for (int r = 0; r < kRows; ++r)
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+      const u32x4* src = reinterpret_cast<const u32x4*>(P.x + (int64_t)row[r] * P.x_stride);
+      const u32x4 v = src[valid(c) ? chunk(c) : 0];
+      raw[r][c] = uint4{v.x, v.y, v.z, v.w};
+    }
+  uint32_t shift[kChunks][4], plus[kChunks][4];   // bf16 pairs: shift and bf16(1 + scale)
+  f32x4 si[kChunks][2];
+  int b = kModulate ? row[0] / P.tokens_per_batch : 0;
+  auto load_modulation = [&]() {
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+      const int at = valid(c) ? chunk(c) : 0;
+      const uint4 sh = reinterpret_cast<const uint4*>(P.shift + (int64_t)b * P.mod_stride)[at];
+      const uint4 sc = reinterpret_cast<const uint4*>(P.scale + (int64_t)b * P.mod_stride)[at];
+      const uint32_t sw[4] = {sh.x, sh.y, sh.z, sh.w}, tw[4] = {sc.x, sc.y, sc.z, sc.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        shift[c][i] = sw[i];
+        plus[c][i] = flk::pack_bf16x2(1.0f + flk::bf16_lo(tw[i]), 1.0f + flk::bf16_hi(tw[i]));
+      }
+    }
+  };
+  if constexpr (kModulate) load_modulation();
 #pragma unroll
   for (int c = 0; c < kChunks; ++c) {
-    const int idx = c * 64 + lane;
-    u32x4 v = {0, 0, 0, 0};
-    if (idx < nch) v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src) + idx);
-    raw[c] = uint4{v.x, v.y, v.z, v.w};
+    const int at = valid(c) ? chunk(c) : 0;
+    si[c][0] = reinterpret_cast<const f32x4*>(P.inv_s)[2 * at];
+    si[c][1] = reinterpret_cast<const f32x4*>(P.inv_s)[2 * at + 1];
   }
-  float xr[kChunks][8];
+  float xr[kRows][kChunks][8];
 #pragma unroll
-  for (int c = 0; c < kChunks; ++c) unpack_bf16x8(raw[c], xr[c]);
+  for (int r = 0; r < kRows; ++r)
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+      if (!valid(c)) raw[r][c] = uint4{0, 0, 0, 0};
+      unpack_bf16x8(raw[r][c], xr[r][c]);
+    }
 
   if constexpr (kModulate) {
-    double sum = 0.0;
+    auto add = [](double p, double q) { return p + q; };
+    const double k = (double)K, rk = 1.0 / k;
+    // v / k, correctly rounded: rk is the rounded reciprocal, so one residual step suffices
+    auto over_k = [&](double v) {
+      const double q = v * rk;
+      return __builtin_fma(__builtin_fma(-q, k, v), rk, q);
+    };
+    double sum[kRows], ssq[kRows];
+    float inv[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      sum[r] = 0.0;
+#pragma unroll
+      for (int c = 0; c < kChunks; ++c)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum[r] += (double)xr[r][c][i];
+    }
+    row_reduce<kRowWaves>(sum, sums, add);
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      const float mean = (float)over_k(sum[r]);
+      ssq[r] = 0.0;
+#pragma unroll
+      for (int c = 0; c < kChunks; ++c)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          xr[r][c][i] = xr[r][c][i] - mean;
+          const float sq = xr[r][c][i] * xr[r][c][i];
+          ssq[r] += (double)(valid(c) ? sq : 0.0f);
+        }
+    }
+    row_reduce<kRowWaves>(ssq, squares, add);
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) inv[r] = 1.0f / sqrtf((float)over_k(ssq[r]) + 1e-6f);
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      if (r > 0) {
+        const int br = row[r] / P.tokens_per_batch;   // wave-uniform
+        if (br != b) {
+          b = br;
+          load_modulation();
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < kChunks; ++c) {
+        uint32_t out[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t base = flk::pack_bf16x2(xr[r][c][2 * i] * inv[r], xr[r][c][2 * i + 1] * inv[r]);
+          const uint32_t prod = flk::pack_bf16x2(flk::bf16_lo(plus[c][i]) * flk::bf16_lo(base),
+                                                 flk::bf16_hi(plus[c][i]) * flk::bf16_hi(base));
+          out[i] = flk::pack_bf16x2(flk::bf16_lo(prod) + flk::bf16_lo(shift[c][i]),
+                                    flk::bf16_hi(prod) + flk::bf16_hi(shift[c][i]));
+          xr[r][c][2 * i] = valid(c) ? flk::bf16_lo(out[i]) : 0.0f;
+          xr[r][c][2 * i + 1] = valid(c) ? flk::bf16_hi(out[i]) : 0.0f;
+        }
+        if (P.x_mod && row0 + r < M && valid(c))
+          reinterpret_cast<uint4*>(P.x_mod + (int64_t)row[r] * P.x_mod_stride)[chunk(c)] =
+              uint4{out[0], out[1], out[2], out[3]};
+      }
+    }
+  }
+
+  float a[kRows];
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) {
+    a[r] = 0.0f;
 #pragma unroll
     for (int c = 0; c < kChunks; ++c)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) sum += (double)xr[c][i];   // padding lanes hold zeros
-    const float mean = (float)(wave_sum(sum) / (double)K);
-    double ssq = 0.0;
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-      const bool valid = c * 64 + lane < nch;
-#pragma unroll
       for (int i = 0; i < 8; ++i) {
-        xr[c][i] = xr[c][i] - mean;
-        if (valid) ssq += (double)(xr[c][i] * xr[c][i]);
+        xr[r][c][i] *= si[c][i >> 2][i & 3];
+        a[r] = fmaxf(a[r], fabsf(xr[r][c][i]));
       }
-    }
-    const float var = (float)(wave_sum(ssq) / (double)K);
-    const float inv = 1.0f / sqrtf(var + 1e-6f);
-    const int b = row / tokens_per_batch;
-    const uint16_t* sh = shift + (int64_t)b * mod_stride;
-    const uint16_t* sc = scale + (int64_t)b * mod_stride;
-    uint16_t* xm = x_mod ? x_mod + (int64_t)row * x_mod_stride : nullptr;
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-      const int idx = c * 64 + lane;
-      if (idx >= nch) continue;
-      float sf[8], tf[8];
-      unpack_bf16x8(*reinterpret_cast<const uint4*>(sh + idx * 8), sf);
-      unpack_bf16x8(*reinterpret_cast<const uint4*>(sc + idx * 8), tf);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float base = flk::round_bf16(xr[c][i] * inv);
-        const float one_plus = flk::round_bf16(1.0f + tf[i]);
-        xr[c][i] = flk::round_bf16(flk::round_bf16(one_plus * base) + sf[i]);
-      }
-      if (xm)
-        *reinterpret_cast<uint4*>(xm + idx * 8) =
-            uint4{flk::pack_bf16x2(xr[c][0], xr[c][1]), flk::pack_bf16x2(xr[c][2], xr[c][3]),
-                  flk::pack_bf16x2(xr[c][4], xr[c][5]), flk::pack_bf16x2(xr[c][6], xr[c][7])};
-    }
   }
-
-  float xh[kChunks][8];
-  float amax = 0.0f;
+  row_reduce<kRowWaves>(a, maxima, [](float p, float q) { return fmaxf(p, q); });
 #pragma unroll
-  for (int c = 0; c < kChunks; ++c) {
-    const int idx = c * 64 + lane;
-    const f32x4 s0 = idx < nch ? reinterpret_cast<const f32x4*>(inv_s)[2 * idx] : f32x4{0, 0, 0, 0};
-    const f32x4 s1 = idx < nch ? reinterpret_cast<const f32x4*>(inv_s)[2 * idx + 1] : f32x4{0, 0, 0, 0};
-    const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+  for (int r = 0; r < kRows; ++r) {
+    if (row0 + r >= M) break;
+    a[r] = absmax_scale(a[r]);
+    const float ra = 1.0f / a[r];
+    uint2* dst = reinterpret_cast<uint2*>(P.xq + (int64_t)row[r] * K);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      xh[c][i] = xr[c][i] * sv[i];
-      amax = fmaxf(amax, fabsf(xh[c][i]));
-    }
+    for (int c = 0; c < kChunks; ++c)
+      if (valid(c)) dst[chunk(c)] = quantize8(xr[r][c], a[r], ra);
+    if (first == 0) P.a_scale[row[r]] = a[r];
   }
-  const float a = absmax_scale(wave_max(amax));
-  const float ra = 1.0f / a;
-  int8_t* dst = xq + (int64_t)row * K;
-#pragma unroll
-  for (int c = 0; c < kChunks; ++c) {
-    const int idx = c * 64 + lane;
-    if (idx < nch) {
-      auto qz = [&](float v) { return quantize_recip(v, a, ra); };
-      uint2 packed;
-      packed.x = pack_i8x4(qz(xh[c][0]), qz(xh[c][1]), qz(xh[c][2]), qz(xh[c][3]));
-      packed.y = pack_i8x4(qz(xh[c][4]), qz(xh[c][5]), qz(xh[c][6]), qz(xh[c][7]));
-      reinterpret_cast<uint2*>(dst)[idx] = packed;
-    }
-  }
-  if (lane == 0) a_scale[row] = a;
 }
 
 // ---------------------------------------------------------------- GEMM -----------------
@@ -1046,20 +1164,30 @@ extern "C" int flk_quantize_weight(const void* w, int64_t w_row_stride, const fl
 
 namespace {
 
+// Waves that share a row of K elements.
+int row_waves(int k) { return k <= 512 ? 1 : k <= 4096 ? 2 : 4; }
+
+#ifndef QROWS
+#define QROWS 1
+#endif
 template <bool kModulate>
 int launch_quantize_act(const QuantGroup& g, int64_t blocks, void* stream) {
   if (blocks > INT32_MAX) return FLK_E_INVALID;
-  const int chunks = (g.K / 8 + 63) / 64;
+  const int waves = row_waves(g.K);
+  const int chunks = (g.K / 8 + 64 * waves - 1) / (64 * waves);
+  const bool full = g.K == 512 * waves * chunks;
   const dim3 grid((unsigned)blocks), block(256);
   const hipStream_t st = as_stream(stream);
-#define FLK_QA(C) hipLaunchKernelGGL((quantize_act_kernel<C, kModulate>), grid, block, 0, st, g)
-  if (chunks <= 1) FLK_QA(1);
-  else if (chunks <= 2) FLK_QA(2);
-  else if (chunks <= 4) FLK_QA(4);
-  else if (chunks <= 6) FLK_QA(6);
-  else if (chunks <= 8) FLK_QA(8);
-  else if (chunks <= 12) FLK_QA(12);
-  else FLK_QA(16);
+#define FLK_QA(W, C) \
+  if (full) hipLaunchKernelGGL((quantize_act_kernel<W, C, true, QROWS, kModulate>), grid, block, 0, st, g); \
+  else hipLaunchKernelGGL((quantize_act_kernel<W, C, false, QROWS, kModulate>), grid, block, 0, st, g)
+  if (waves == 1) { FLK_QA(1, 1); }
+  else if (waves == 2 && chunks == 1) { FLK_QA(2, 1); }
+  else if (waves == 2 && chunks == 2) { FLK_QA(2, 2); }
+  else if (waves == 2 && chunks == 3) { FLK_QA(2, 3); }
+  else if (waves == 2) { FLK_QA(2, 4); }
+  else if (chunks <= 3) { FLK_QA(4, 3); }
+  else { FLK_QA(4, 4); }
 #undef FLK_QA
   return flk_launch_status();
 }
@@ -1089,7 +1217,10 @@ int modulated_problem(const void* x, int64_t x_row_stride, const void* shift, co
   return FLK_OK;
 }
 
-int64_t row_blocks(const QuantProblem& p) { return ((int64_t)p.M + 3) / 4; }
+int64_t row_blocks(const QuantProblem& p, int k) {
+  const int rows = 4 / row_waves(k) * QROWS;
+  return ((int64_t)p.M + rows - 1) / rows;
+}
 
 }  // namespace
 
@@ -1105,7 +1236,7 @@ extern "C" int flk_quantize_act(const void* x, int64_t x_row_stride, const float
     return FLK_E_ALIGN;
   const QuantProblem p{static_cast<const uint16_t*>(x), x_row_stride, inv_s, m, xq, a_scale, nullptr, nullptr, 0, 1,
                        nullptr, 0};
-  const int64_t blocks = row_blocks(p);
+  const int64_t blocks = row_blocks(p, k);
   return launch_quantize_act<false>(QuantGroup{{p, p}, (int)std::min<int64_t>(blocks, INT32_MAX), k}, blocks,
                                     stream);
 }
@@ -1118,7 +1249,7 @@ extern "C" int flk_quantize_act_modulated(const void* x, int64_t x_row_stride, c
   const int st = modulated_problem(x, x_row_stride, shift, scale, mod_batch_stride, tokens_per_batch, inv_s, m, k,
                                    xq, a_scale, x_mod, x_mod_row_stride, p);
   if (st != FLK_OK) return st == kNoWork ? FLK_OK : st;
-  const int64_t blocks = row_blocks(p);
+  const int64_t blocks = row_blocks(p, k);
   return launch_quantize_act<true>(QuantGroup{{p, p}, (int)std::min<int64_t>(blocks, INT32_MAX), k}, blocks,
                                    stream);
 }
@@ -1143,8 +1274,8 @@ extern "C" int flk_quantize_act_modulated_pair(
   if (st0 == kNoWork) g.p[0] = g.p[1];
   if (st1 == kNoWork) g.p[1] = g.p[0];
   const bool both = st0 == FLK_OK && st1 == FLK_OK;
-  const int64_t b0 = row_blocks(g.p[0]);
-  const int64_t blocks = both ? b0 + row_blocks(g.p[1]) : b0;
+  const int64_t b0 = row_blocks(g.p[0], k);
+  const int64_t blocks = both ? b0 + row_blocks(g.p[1], k) : b0;
   g.first_blocks = (int)std::min<int64_t>(b0, INT32_MAX);
   return launch_quantize_act<true>(g, blocks, stream);
 }

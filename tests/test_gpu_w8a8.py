@@ -438,6 +438,37 @@ def test_modulated_activation_bit_exact(device, batch, length, k):
     assert torch.equal(xq2, xq) and torch.equal(a2, a_scale)
 
 
+@pytest.mark.parametrize("k", [8, 504, 512, 520, 1024, 1032, 2048, 3072, 3080, 4096, 4104, 6144, 6152, 8192])
+def test_quantize_act_widths(device, k):
+    """Each split of a row over waves and chunks, full and ragged, with a last block that is not
+    full; rows of zeros, of values whose scale is subnormal (1 / a overflows) or small, and of
+    one infinity (0 for the finite values).  Codes and scales bit for bit."""
+    rng = np.random.default_rng(k)
+    x = rng.standard_normal((7, k)).astype(np.float32)
+    x[1] = 0.0
+    x[2] *= 1e-38
+    x[3] *= 2e-37
+    x[4, k // 2] = 3e4
+    x = torch.from_numpy(x).to(torch.bfloat16)
+    inv = (0.5 + rng.random(k)).astype(np.float32)
+    xq_want, a_want = Q.quantize_act(x.float().numpy(), inv)
+    xi = x.clone()
+    xi[6, 0] = float("inf")
+    xq, a = w8a8.quantize_act(xi.to(device), torch.from_numpy(inv).to(device))
+    np.testing.assert_array_equal(host(a)[:6], a_want[:6])
+    np.testing.assert_array_equal(host(xq)[:6], xq_want[:6])
+    assert host(a)[6] == np.inf and not host(xq)[6, 1:].any()
+    shift, scale = (torch.from_numpy(0.3 * rng.standard_normal((1, k)).astype(np.float32)).to(torch.bfloat16)
+                    for _ in range(2))
+    mq, ma, mx = w8a8.quantize_act_modulated(x[None].to(device), shift.to(device), scale.to(device),
+                                             torch.from_numpy(inv).to(device), x_mod=True)
+    want = Q.modulate(host_f32(x[None]), host_f32(shift), host_f32(scale))
+    assert_bits_equal(mx, want, "modulated X")
+    want_q, want_a = Q.quantize_act(want.reshape(-1, k), inv)
+    np.testing.assert_array_equal(host(mq), want_q)
+    np.testing.assert_array_equal(host(ma), want_a)
+
+
 def test_modulated_projection_qk_prep(device):
     """The whole qkv_prep(linear(modulate(x, mod1), w), ...) of a block in two launches equals
     the step-by-step path (modulated X, then the fused projection + qk_prep)."""
