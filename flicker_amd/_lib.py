@@ -26,6 +26,8 @@ SIGNATURES = {
     "flk_qk_prep_f32": (_i, [_p, _i64, _i64, _p, _p, _i64, _p, _p, _i, _i, _i, _i, _p, _p, _p, _i64, _i64, _p]),
     "flk_qk_prep_ids": (_i, [_p, _i64, _i64, _p, _i64, _i, _ip, _f, _p, _p, _i, _f, _i, _i, _i, _i,
                              _p, _p, _p, _i64, _i64, _p]),
+    "flk_qk_prep_pair": (_i, [_p, _i64, _i64, _p, _p, _p, _p, _i, _i64, _p, _i64, _i64, _p, _p, _p, _p, _i, _i64,
+                              _i64, _i, _f, _i, _i, _i, _p, _p, _p, _i64, _p]),
     "flk_attend": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _p]),
     "flk_attend_to": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i64, _i64, _i64, _p]),
     "flk_attend_split_to": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i64, _i64, _i64, _i, _p, _i64, _p]),

@@ -97,14 +97,15 @@ __device__ __forceinline__ void store_f32x8(float* p, const float r[8]) {
 
 // kOutF32: q and k are stored as float32 (no gain, no final rounding): the plain branch of
 // qkv_prep with float32 scales (flk_qk_prep_f32); q_out / k_out then point at floats.
-template <bool kScaleF32, bool kGain, int kHeads, bool kOutF32 = false>
-__global__ __launch_bounds__(kThreads) void qk_prep_kernel(
-    const uint16_t* __restrict__ qkv, int64_t batch_stride, int64_t row_stride, RopeSource rope,
+// block: the token block, kTokensPerBlock tokens of every head group and batch entry.
+template <bool kScaleF32, bool kGain, int kHeads, bool kOutF32>
+__device__ __forceinline__ void qk_prep_rows(
+    const uint16_t* __restrict__ qkv, int64_t batch_stride, int64_t row_stride, const RopeSource& rope,
     const void* __restrict__ q_scale, const void* __restrict__ k_scale, float q_gain,
     int length, int num_heads, uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out,
-    uint16_t* __restrict__ v_out, int64_t out_length, int64_t out_offset) {
+    uint16_t* __restrict__ v_out, int64_t out_length, int64_t out_offset, int block) {
   const int lane = threadIdx.x & (kLanesPerRow - 1);
-  const int t = blockIdx.x * kTokensPerBlock + (threadIdx.x >> 4);
+  const int t = block * kTokensPerBlock + (threadIdx.x >> 4);
   if (t >= length) return;  // whole 16-lane rows exit together, so DPP rows stay intact
   const int h0 = blockIdx.y * kHeads;
   const int b = blockIdx.z;
@@ -139,6 +140,54 @@ __global__ __launch_bounds__(kThreads) void qk_prep_kernel(
     }
     store16(v_out + o, rv[i]);
   }
+}
+
+template <bool kScaleF32, bool kGain, int kHeads, bool kOutF32 = false>
+__global__ __launch_bounds__(kThreads) void qk_prep_kernel(
+    const uint16_t* __restrict__ qkv, int64_t batch_stride, int64_t row_stride, RopeSource rope,
+    const void* __restrict__ q_scale, const void* __restrict__ k_scale, float q_gain,
+    int length, int num_heads, uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out,
+    uint16_t* __restrict__ v_out, int64_t out_length, int64_t out_offset) {
+  qk_prep_rows<kScaleF32, kGain, kHeads, kOutF32>(qkv, batch_stride, row_stride, rope, q_scale, k_scale, q_gain,
+                                                  length, num_heads, q_out, k_out, v_out, out_length, out_offset,
+                                                  blockIdx.x);
+}
+
+// Both streams of a double block in one launch (tables form, two heads per group): token blocks
+// [0, first_blocks) of the grid's x take p[0], the rest p[1].  The text stream's 64 token blocks
+// alone leave most of the chip idle, and each launch costs the caller its own call.
+struct PairStream {
+  const uint16_t* qkv;
+  int64_t batch_stride, row_stride;
+  const float* cos;
+  const float* sin;
+  const void* q_scale;
+  const void* k_scale;
+  int length;
+  int64_t out_offset;
+};
+
+struct PairLaunch {
+  PairStream p[2];
+  int first_blocks;
+  int64_t table_stride;
+  float q_gain;
+  int num_heads;
+  uint16_t *q, *k, *v;
+  int64_t out_length;
+};
+
+template <bool kScaleF32, int kHeads>
+__global__ __launch_bounds__(kThreads) void qk_prep_pair_kernel(const PairLaunch a) {
+  const bool second = (int)blockIdx.x >= a.first_blocks;
+  const PairStream& P = second ? a.p[1] : a.p[0];   // wave-uniform, read from the kernel arguments
+  RopeSource rope{};
+  rope.cos = P.cos;
+  rope.sin = P.sin;
+  rope.table_stride = a.table_stride;
+  qk_prep_rows<kScaleF32, true, kHeads, false>(P.qkv, P.batch_stride, P.row_stride, rope, P.q_scale, P.k_scale,
+                                                a.q_gain, P.length, a.num_heads, a.q, a.k, a.v, a.out_length,
+                                                P.out_offset, (int)blockIdx.x - (second ? a.first_blocks : 0));
 }
 
 // The ids form.  Each 16-lane group computes the cos / sin of its 4 pairs once and applies
@@ -426,4 +475,54 @@ extern "C" int flk_qk_prep_ids(const void* qkv, int64_t qkv_batch_stride, int64_
   a.out_offset = out_offset;
   return dispatch<true>(heads_per_group(num_heads, true, FLK_QK_IDS_HPG), batch, scale_is_f32,
                         static_cast<hipStream_t>(stream), a);
+}
+
+extern "C" int flk_qk_prep_pair(const void* qkv0, int64_t qkv_batch_stride0, int64_t qkv_row_stride0,
+                                const float* cos0, const float* sin0, const void* q_scale0, const void* k_scale0,
+                                int length0, int64_t out_offset0, const void* qkv1, int64_t qkv_batch_stride1,
+                                int64_t qkv_row_stride1, const float* cos1, const float* sin1, const void* q_scale1,
+                                const void* k_scale1, int length1, int64_t out_offset1, int64_t table_row_stride,
+                                int scale_is_f32, float q_gain, int batch, int num_heads, int head_dim, void* q_out,
+                                void* k_out, void* v_out, int64_t out_length, void* stream) {
+  const PairStream streams[2] = {{static_cast<const uint16_t*>(qkv0), qkv_batch_stride0, qkv_row_stride0, cos0, sin0,
+                                  q_scale0, k_scale0, length0, out_offset0},
+                                 {static_cast<const uint16_t*>(qkv1), qkv_batch_stride1, qkv_row_stride1, cos1, sin1,
+                                  q_scale1, k_scale1, length1, out_offset1}};
+  PairLaunch a{};
+  int n = 0;   // streams with work; an empty one is left out
+  for (const PairStream& p : streams) {
+    const int st = check_common(p.qkv, p.batch_stride, p.row_stride, p.q_scale, p.k_scale, batch, p.length, num_heads,
+                                head_dim, q_out, k_out, v_out, out_length, p.out_offset);
+    if (st == kEmpty) continue;
+    if (st != FLK_OK) return st;
+    if (table_row_stride < head_dim || !p.cos || !p.sin) return FLK_E_INVALID;
+    if (table_row_stride % 4 || !flk_host_aligned(p.cos, 16) || !flk_host_aligned(p.sin, 16)) return FLK_E_ALIGN;
+    a.p[n++] = p;
+  }
+  if (n == 0) return FLK_OK;
+  if (n == 1) a.p[1] = a.p[0];
+  auto blocks = [](const PairStream& p) { return ((int64_t)p.length + kTokensPerBlock - 1) / kTokensPerBlock; };
+  const int64_t first = blocks(a.p[0]), total = first + (n == 2 ? blocks(a.p[1]) : 0);
+  a.first_blocks = (int)first;
+  a.table_stride = table_row_stride;
+  a.q_gain = q_gain;
+  a.num_heads = num_heads;
+  a.q = static_cast<uint16_t*>(q_out);
+  a.k = static_cast<uint16_t*>(k_out);
+  a.v = static_cast<uint16_t*>(v_out);
+  a.out_length = out_length;
+  const int hpg = num_heads % 2 == 0 ? 2 : 1;
+  const dim3 grid((unsigned)total, num_heads / hpg, batch);
+  const hipStream_t hs = static_cast<hipStream_t>(stream);
+#define FLK_QK_PAIR(F32, NH) \
+  hipLaunchKernelGGL((qk_prep_pair_kernel<F32, NH>), grid, dim3(kThreads), 0, hs, a)
+  if (hpg == 2) {
+    if (scale_is_f32) FLK_QK_PAIR(true, 2);
+    else FLK_QK_PAIR(false, 2);
+  } else {
+    if (scale_is_f32) FLK_QK_PAIR(true, 1);
+    else FLK_QK_PAIR(false, 1);
+  }
+#undef FLK_QK_PAIR
+  return flk_launch_status();
 }

@@ -138,12 +138,10 @@ def _id_args(pos: PositionIds, length: int, head_dim: int):
     return ids if ids.stride(1) == 1 else ids.contiguous()
 
 
-def _launch_qk_prep(qkv, q_scale, k_scale, freqs, num_heads: int, out, out_offset: int,
-                    qk_f32: bool = False):
-    """qk_prep's launch.  ``qk_f32``: the plain branch of qkv_prep with float32 scales
-    (modules.py:78-80, where rms_norm's product and apply_rope's result stay float32): q and
-    k come out float32, unrounded and without a query gain (flk_qk_prep_f32); v stays bf16."""
-    batch, length, width = qkv.shape
+def _qk_operands(qkv, q_scale, k_scale, freqs, num_heads: int, qk_f32: bool = False):
+    """Checked operands of one stream: (qkv, q_scale, k_scale, RoPE source, its device operands,
+    head_dim)."""
+    _, length, width = qkv.shape
     head_dim = width // (3 * num_heads)
     if 3 * num_heads * head_dim != width:
         raise ValueError(f"qkv width {width} is not 3 * num_heads({num_heads}) * head_dim")
@@ -158,19 +156,38 @@ def _launch_qk_prep(qkv, q_scale, k_scale, freqs, num_heads: int, out, out_offse
         rope = _table_args(freqs, length, head_dim)
     else:
         raise TypeError(f"freqs must be Freqs or PositionIds, got {type(freqs).__name__}")
-    q_gain = freqs.q_gain
     _on_gpu("q_scale", q_scale)
     _on_gpu("k_scale", k_scale)
     if q_scale.numel() != head_dim or k_scale.numel() != head_dim:
         raise ValueError(f"q_scale / k_scale must hold {head_dim} values")
     if q_scale.dtype != k_scale.dtype or q_scale.dtype not in (torch.bfloat16, torch.float32):
         raise TypeError("q_scale and k_scale must share one dtype, bfloat16 or float32")
-    if qk_f32 and (q_scale.dtype != torch.float32 or isinstance(freqs, PositionIds) or q_gain != 1.0):
+    if qk_f32 and (q_scale.dtype != torch.float32 or isinstance(freqs, PositionIds) or freqs.q_gain != 1.0):
         raise ValueError("float32 q / k outputs are the plain branch's: float32 scales, lane tables, gain 1")
-    qk_dtype = torch.float32 if qk_f32 else torch.bfloat16
     qkv = _dense_rows(qkv)
     q_scale, k_scale = _vector(q_scale), _vector(k_scale)
+    return qkv, q_scale, k_scale, freqs, rope, head_dim
 
+
+def _qk_outputs(out, batch: int, num_heads: int, out_length: int, head_dim: int, qk_dtype):
+    """Checks an (q, k, v) output triple of (B, H, out_length, D) tensors."""
+    shape = (batch, num_heads, out_length, head_dim)
+    for t, dt in zip(out, (qk_dtype, qk_dtype, torch.bfloat16)):
+        _on_gpu("out", t)
+        if t.dtype != dt or t.shape != shape or not t.is_contiguous():
+            raise ValueError(f"out tensors must be contiguous (B, H, L_out, D) of one shape, q and k "
+                             f"{qk_dtype}, v bfloat16")
+
+
+def _launch_qk_prep(qkv, q_scale, k_scale, freqs, num_heads: int, out, out_offset: int,
+                    qk_f32: bool = False):
+    """qk_prep's launch.  ``qk_f32``: the plain branch of qkv_prep with float32 scales
+    (modules.py:78-80, where rms_norm's product and apply_rope's result stay float32): q and
+    k come out float32, unrounded and without a query gain (flk_qk_prep_f32); v stays bf16."""
+    batch, length, _ = qkv.shape
+    qkv, q_scale, k_scale, freqs, rope, head_dim = _qk_operands(qkv, q_scale, k_scale, freqs, num_heads, qk_f32)
+    q_gain = freqs.q_gain
+    qk_dtype = torch.float32 if qk_f32 else torch.bfloat16
     if out is None:
         if out_offset:
             raise ValueError("out_offset needs out=(q, k, v)")
@@ -183,12 +200,7 @@ def _launch_qk_prep(qkv, q_scale, k_scale, freqs, num_heads: int, out, out_offse
         if len(out) != 3:
             raise ValueError("out must be a (q, k, v) triple")
         out_length = out[0].shape[2]
-        shape = (batch, num_heads, out_length, head_dim)
-        for t, dt in zip(out, (qk_dtype, qk_dtype, torch.bfloat16)):
-            _on_gpu("out", t)
-            if t.dtype != dt or t.shape != shape or not t.is_contiguous():
-                raise ValueError(f"out tensors must be contiguous (B, H, L_out, D) of one shape, q and k "
-                                 f"{qk_dtype}, v bfloat16")
+        _qk_outputs(out, batch, num_heads, out_length, head_dim, qk_dtype)
         if out_offset < 0 or out_offset + length > out_length:
             raise ValueError(f"out_offset {out_offset} + L {length} exceeds the output length {out_length}")
 
@@ -211,6 +223,27 @@ def _launch_qk_prep(qkv, q_scale, k_scale, freqs, num_heads: int, out, out_offse
         cos, sin = rope
         _lib.run("flk_qk_prep", (qkv, cos, sin, q_scale, k_scale, *out),
                  qkv.data_ptr(), *qkv.stride()[:2], cos.data_ptr(), sin.data_ptr(), cos.stride(0), *common)
+    return out
+
+
+def _launch_qk_prep_pair(txt, img, num_heads: int, out):
+    """qk_prep's launch of both streams of a double block, each (qkv, q_scale, k_scale, Freqs), into
+    the joint (q, k, v) ``out``, text first (flk_qk_prep_pair).  The streams must share their
+    scales' dtype, q_gain and batch; lane tables of another row stride are compacted."""
+    streams = []
+    for qkv, q_scale, k_scale, freqs in (txt, img):
+        qkv, q_scale, k_scale, freqs, (cos, sin), head_dim = _qk_operands(qkv, q_scale, k_scale, freqs, num_heads)
+        if cos.stride(0) != head_dim:
+            cos, sin = cos.contiguous(), sin.contiguous()
+        streams.append((qkv, cos, sin, q_scale, k_scale))
+    batch, len0, _ = txt[0].shape
+    len1 = img[0].shape[1]
+    args = []
+    for (qkv, *rest), length, offset in zip(streams, (len0, len1), (0, len0)):
+        args += [qkv.data_ptr(), *qkv.stride()[:2], *(t.data_ptr() for t in rest), length, offset]
+    _lib.run("flk_qk_prep_pair", (*streams[0], *streams[1], *out), *args, head_dim,
+             int(streams[0][3].dtype == torch.float32), float(txt[3].q_gain), batch, num_heads, head_dim,
+             out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(), len0 + len1, _lib.stream_of(out[0]))
     return out
 
 

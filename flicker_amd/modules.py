@@ -12,7 +12,7 @@ from __future__ import annotations
 
 import torch
 
-from .kernels import Freqs, PositionIds, _launch_qk_prep, attend_merged, lane_pair, row_tile
+from .kernels import Freqs, PositionIds, _launch_qk_prep, _launch_qk_prep_pair, attend_merged, lane_pair, row_tile
 
 
 def heads(qkv: torch.Tensor, num_heads: int):
@@ -77,8 +77,9 @@ def double_attention(txt_qkv, img_qkv, txt_scales, img_scales, freqs: Freqs | Po
     """modules.py:127-139 + 157-158 -- per-stream qk prep, joint text|image attention, merge,
     split back into (txt_attn, img_attn), each (B, L_stream, H*D).
 
-    Both qk_prep calls write into one (B, H, L_txt + L_img, D) buffer at their sequence
-    offsets, which replaces the reference's three concatenations.  ``pe_ctx`` / ``pe`` are the
+    Both streams' qk prep writes into one (B, H, L_txt + L_img, D) buffer at their sequence
+    offsets, which replaces the reference's three concatenations -- in one launch when both
+    take the fused form from lane tables with scales of one dtype.  ``pe_ctx`` / ``pe`` are the
     text / image rope tables the reference hands each stream's qkv_prep (modules.py:129,133);
     they are read only by a stream whose length has no row tile (the gate's plain branch)."""
     batch, num_txt, width = txt_qkv.shape
@@ -90,9 +91,14 @@ def double_attention(txt_qkv, img_qkv, txt_scales, img_scales, freqs: Freqs | Po
     head_dim = width // (3 * num_heads)
     shape = (batch, num_heads, num_txt + num_img, head_dim)
     joint = tuple(torch.empty(shape, dtype=torch.bfloat16, device=txt_qkv.device) for _ in range(3))
-    qkv_prep(txt_qkv, *txt_scales, pe_ctx, _slice(freqs, 0, num_txt), num_heads, out=joint, out_offset=0)
-    qkv_prep(img_qkv, *img_scales, pe, _slice(freqs, num_txt, num_txt + num_img), num_heads,
-             out=joint, out_offset=num_txt)
+    if (isinstance(freqs, Freqs) and row_tile(num_txt) is not None and row_tile(num_img) is not None
+            and txt_scales[0].dtype == img_scales[0].dtype and img_qkv.shape[0] == batch):
+        _launch_qk_prep_pair((txt_qkv, *txt_scales, _slice(freqs, 0, num_txt)),
+                             (img_qkv, *img_scales, _slice(freqs, num_txt, num_txt + num_img)), num_heads, joint)
+    else:
+        qkv_prep(txt_qkv, *txt_scales, pe_ctx, _slice(freqs, 0, num_txt), num_heads, out=joint, out_offset=0)
+        qkv_prep(img_qkv, *img_scales, pe, _slice(freqs, num_txt, num_txt + num_img), num_heads,
+                 out=joint, out_offset=num_txt)
     attn = attend_merged(*joint)   # merge_heads fused into the attention epilogue
     return attn[:, :num_txt], attn[:, num_txt:]
 

@@ -101,6 +101,22 @@ int flk_qk_prep_ids(const void* qkv, int64_t qkv_batch_stride, int64_t qkv_row_s
                     int64_t out_offset, void* stream);
 
 /*
+ * flk_qk_prep of both streams of a double block (src/flicker/modules.py:127-139: each stream's
+ * qkv_prep, then the text | image concatenations) in one launch: stream i writes its rows at
+ * out_offset_i of the joint outputs, the bits of its own flk_qk_prep.  Arguments as flk_qk_prep;
+ * batch, heads, table_row_stride, the scales' type and q_gain are the streams' common ones.  An
+ * empty stream (length 0) is skipped; a refused one refuses the call before any launch.
+ */
+int flk_qk_prep_pair(const void* qkv0, int64_t qkv_batch_stride0, int64_t qkv_row_stride0,
+                     const float* cos0, const float* sin0, const void* q_scale0, const void* k_scale0,
+                     int length0, int64_t out_offset0,
+                     const void* qkv1, int64_t qkv_batch_stride1, int64_t qkv_row_stride1,
+                     const float* cos1, const float* sin1, const void* q_scale1, const void* k_scale1,
+                     int length1, int64_t out_offset1,
+                     int64_t table_row_stride, int scale_is_f32, float q_gain, int batch, int num_heads,
+                     int head_dim, void* q_out, void* k_out, void* v_out, int64_t out_length, void* stream);
+
+/*
  * Bounded flash attention: softmax without the running max, legal because the
  * QK-norm scales bound every logit (checked at load time, kernels.logit_bound).
  * Replaces kernels.attend (src/flicker/kernels.py:105-145).

@@ -309,3 +309,31 @@ def test_qk_prep_random_shapes(device):
         want = P.qk_prep_fused(to_np(qkv), to_np(qs), to_np(ks), lanes, heads, scale_is_bf16=not f32,
                                return_normed=True)
         check_qkv(label, via_tables, want, gain)
+
+
+@pytest.mark.parametrize("batch,len0,len1,heads,scale_dtype,gain", [
+    (1, 512, 256, 24, torch.bfloat16, 128 ** -0.5),
+    (2, 1, 130, 3, torch.float32, 0.3),             # odd heads, token blocks that are not full
+    (2, 7, 8, 2, torch.bfloat16, 1.0),
+    (1, 0, 64, 4, torch.bfloat16, 0.5),             # an empty stream
+    (3, 65, 0, 5, torch.bfloat16, 0.5),
+])
+def test_pair_equals_two_launches(device, batch, len0, len1, heads, scale_dtype, gain):
+    """flk_qk_prep_pair writes the bits of each stream's own flk_qk_prep at its offset, from a
+    strided activation and tables of a wider row stride as from dense ones."""
+    g = torch.Generator().manual_seed(len0 + 3 * len1)
+    streams = []
+    for i, n in enumerate((len0, len1)):
+        wide = torch.randn(batch, n, 3 * heads * D + 64, generator=g).to(torch.bfloat16).to(device)
+        qkv = wide[..., :3 * heads * D] if i else wide[..., :3 * heads * D].contiguous()
+        qs, ks = ((1 + 0.1 * torch.randn(D, generator=g)).to(scale_dtype).to(device) for _ in range(2))
+        tables = torch.randn(2, n, D + 4 * i, generator=g).to(device)[..., :D]
+        streams.append((qkv, qs, ks, kernels.Freqs(tables[0], tables[1], gain)))
+    shape = (batch, heads, len0 + len1, D)
+    want, got = (tuple(torch.full(shape, 5.0, dtype=torch.bfloat16, device=device) for _ in range(3)) for _ in range(2))
+    kernels._launch_qk_prep(*streams[0], heads, want, 0)
+    kernels._launch_qk_prep(*streams[1], heads, want, len0)
+    kernels._launch_qk_prep_pair(*streams, heads, got)
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
