@@ -34,6 +34,8 @@ SIGNATURES = {
     "flk_attend_split_static_to": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i64, _i64, _i64, _i, _p]),
     "flk_attend_balanced_to": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i64, _i64, _i64, _p, _i64, _p]),
     "flk_attend_balanced_plan": (_i, [_i, _i, _i, _ip, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64)]),
+    "flk_attend_halves_plan": (_i, [_i, _i, _i, _ip]),
+    "flk_attend_halves_to": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i64, _i64, _i64, _i, _p]),
     "flk_attend_plan": (_i, [_i, _i, _i, _ip, ctypes.POINTER(ctypes.c_int64)]),
     "flk_attend_kernel": (ctypes.c_char_p, [_i, _i, _i]),
     "flk_rope_embed": (_i, [_p, _i64, _i64, _i, _ip, _f, _p, _p]),
@@ -167,6 +169,15 @@ def attend_balanced_plan(batch: int, heads: int, length: int) -> tuple[int, int,
     check(lib().flk_attend_balanced_plan(batch, heads, length, ctypes.byref(grid), ctypes.byref(nbytes),
                                          ctypes.byref(off)), "flk_attend_balanced_plan")
     return grid.value, nbytes.value, off.value
+
+
+@functools.lru_cache(maxsize=1024)
+def attend_halves_plan(batch: int, heads: int, length: int) -> int:
+    """Queries per block of flk_attend_halves_to for a shape, or 0 where another launch is chosen (a
+    pure function of the shape)."""
+    queries = ctypes.c_int(0)
+    check(lib().flk_attend_halves_plan(batch, heads, length, ctypes.byref(queries)), "flk_attend_halves_plan")
+    return queries.value
 
 
 _BALANCED_WORKSPACE: dict = {}

@@ -263,11 +263,12 @@ struct TileCopy {
   uint32_t off[kDmaPerTensor];
 };
 
+template <int kRows = kBN>
 __device__ __forceinline__ TileCopy plan_copy(uint8_t* dst, const uint16_t* __restrict__ head, int tile,
                                               const CopyPlan& cp) {
   tile = min(tile, cp.last_tile);
   TileCopy tc;
-  tc.base = head + (int64_t)tile * kBN * kD;
+  tc.base = head + (int64_t)tile * kRows * kD;
   tc.dst = dst + cp.lds_wave_off;
   const bool last = tile == cp.last_tile;
 #pragma unroll
@@ -280,9 +281,10 @@ __device__ __forceinline__ void issue_copy(const TileCopy& tc, int i) {
 }
 
 // Copy 64-key tile `tile` (clamped to the last one) of K or V into an LDS ring slot at once.
+template <int kRows = kBN>
 __device__ __forceinline__ void copy_tile(uint8_t* dst, const uint16_t* __restrict__ head, int tile,
                                           const CopyPlan& cp) {
-  const TileCopy tc = plan_copy(dst, head, tile, cp);
+  const TileCopy tc = plan_copy<kRows>(dst, head, tile, cp);
 #pragma unroll
   for (int i = 0; i < kDmaPerTensor; ++i) issue_copy(tc, i);
 }
@@ -338,6 +340,62 @@ __device__ __forceinline__ void iteration(WaveState<G>& w, const Ctx& c, int t, 
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(kDmaPerIter) : "memory");
 }
 
+// Loads the wave's 16 G queries from q0 of a head and sets its accumulators, operand offsets and
+// P(-1).  unit_off: bytes added to every K and V operand offset.
+template <int G>
+__device__ __forceinline__ void start_wave(WaveState<G>& w, const uint16_t* __restrict__ qh, int q0, int length,
+                                           int unit_off) {
+  const int lane = threadIdx.x & 63;
+  const int h = lane >> 4, col = lane & 15;
+  // k-slots 8h..8h+7 of the S MFMAs take d chunk dperm = 4 st + perm(h) of the K and Q rows,
+  // perm(h) = 0, 2, 1, 3: lanes l and l + 32 then read neighbouring chunks (c, c ^ 1), which
+  // the swizzle keeps on distinct banks whether a b128 read is served as 16 consecutive lanes
+  // or as 8 lanes from each half of the wave.
+  const int hperm = ((h & 1) << 1) | (h >> 1);
+#pragma unroll
+  for (int g = 0; g < G; ++g) {   // query group g of this wave: q0 + 16 g .. + 15
+    const int qi = q0 + g * 16 + col;
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+      w.qreg[st][g] = qi < length
+                          ? *reinterpret_cast<const bf16x8*>(qh + (int64_t)qi * kD + st * 32 + hperm * 8)
+                          : bf16x8{};
+  }
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+    for (int g = 0; g < G; ++g) w.oacc[dt][g] = f32x4{};
+#pragma unroll
+  for (int g = 0; g < G; ++g) w.lacc[g] = f32x4{};
+  {
+    const __bf16 one = (lane & 15) == 0 ? (__bf16)1.0f : (__bf16)0.0f;
+    w.ones = bf16x8{one, one, one, one, one, one, one, one};
+  }
+#pragma unroll
+  for (int st = 0; st < 4; ++st) {
+    // K operand of d step st: row col of the 16-key tile, d = 32 st + 8 perm(h) .. +7
+    w.k_off[st] = unit_off + kKRing + col * kRowBytes + ((((st << 2) | hperm) ^ swz(col)) << 4);
+    asm volatile("" : "+v"(w.k_off[st]));
+  }
+  {
+    // Transpose-read source lane sl of lane group h -> key 4h + sl/4 (+16 for k-slots 4-7),
+    // columns 16 dt + 4 (sl % 4) .. +3: chunk 2 dt + (sl % 4) / 2, half sl % 2.
+    const int sl = lane & 15;
+    const int key = h * 4 + (sl >> 2);
+    const int half = sl & 1;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) {
+      const int chunk = 2 * dt + ((sl & 3) >> 1);
+      w.v_off[dt] = unit_off + key * kRowBytes + ((chunk ^ swz(key)) << 4) + half * 8;
+      // Opaque to the compiler: it then adds the (immediate) unit offsets with the DS
+      // instruction's offset field instead of a v_or per read.
+      asm volatile("" : "+v"(w.v_off[dt]));
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4 * G; ++i) w.pB[i] = 0u;   // P(-1) = 0: phase 0's PV MFMAs add nothing
+}
+
 // One segment of work for a block: head bh (batch-major), key tiles [t_begin, t_end), and
 // for this wave the 16 G queries from q0.  On return w holds the segment's unnormalised O^T accumulators and row
 // sums (lacc), and every LDS read and copy of the segment has completed.  Ring slots count from
@@ -352,7 +410,6 @@ __device__ __forceinline__ void attend_segment(WaveState<G>& w, uint8_t* smem, c
   Ctx c;
   c.smem = smem;
   c.h = lane >> 4;            // lane group: k-slots 8h..8h+7 and accumulator rows 4h..4h+3
-  const int col = lane & 15;  // query column (S^T, O^T) / operand row (K, V^T) in a 16-tile
   c.length = length;
   c.ntiles = (length + kBN - 1) / kBN;
   c.cp.last_tile = c.ntiles - 1;
@@ -378,53 +435,7 @@ __device__ __forceinline__ void attend_segment(WaveState<G>& w, uint8_t* smem, c
   for (int tl = 0; tl < 3; ++tl) copy_tile(smem + kKRing + tl * kTileBytes, c.kh, t_begin + tl, c.cp);
   for (int tl = 0; tl < 2; ++tl) copy_tile(smem + kVRing + tl * kTileBytes, c.vh, t_begin + tl, c.cp);
 
-  // k-slots 8h..8h+7 of the S MFMAs take d chunk dperm = 4 st + perm(h) of the K and Q rows,
-  // perm(h) = 0, 2, 1, 3: lanes l and l + 32 then read neighbouring chunks (c, c ^ 1), which
-  // the swizzle keeps on distinct banks whether a b128 read is served as 16 consecutive lanes
-  // or as 8 lanes from each half of the wave.
-  const int hperm = ((c.h & 1) << 1) | (c.h >> 1);
-#pragma unroll
-  for (int g = 0; g < G; ++g) {   // query group g of this wave: q0 + 16 g .. + 15
-    const int qi = q0 + g * 16 + col;
-#pragma unroll
-    for (int st = 0; st < 4; ++st)
-      w.qreg[st][g] = qi < length
-                          ? *reinterpret_cast<const bf16x8*>(qh + (int64_t)qi * kD + st * 32 + hperm * 8)
-                          : bf16x8{};
-  }
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-    for (int g = 0; g < G; ++g) w.oacc[dt][g] = f32x4{};
-#pragma unroll
-  for (int g = 0; g < G; ++g) w.lacc[g] = f32x4{};
-  {
-    const __bf16 one = (lane & 15) == 0 ? (__bf16)1.0f : (__bf16)0.0f;
-    w.ones = bf16x8{one, one, one, one, one, one, one, one};
-  }
-#pragma unroll
-  for (int st = 0; st < 4; ++st) {
-    // K operand of d step st: row col of the 16-key tile, d = 32 st + 8 perm(h) .. +7
-    w.k_off[st] = kKRing + col * kRowBytes + ((((st << 2) | hperm) ^ swz(col)) << 4);
-    asm volatile("" : "+v"(w.k_off[st]));
-  }
-  {
-    // Transpose-read source lane sl of lane group h -> key 4h + sl/4 (+16 for k-slots 4-7),
-    // columns 16 dt + 4 (sl % 4) .. +3: chunk 2 dt + (sl % 4) / 2, half sl % 2.
-    const int sl = lane & 15;
-    const int key = c.h * 4 + (sl >> 2);
-    const int half = sl & 1;
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      const int chunk = 2 * dt + ((sl & 3) >> 1);
-      w.v_off[dt] = key * kRowBytes + ((chunk ^ swz(key)) << 4) + half * 8;
-      // Opaque to the compiler: it then adds the (immediate) unit offsets with the DS
-      // instruction's offset field instead of a v_or per read.
-      asm volatile("" : "+v"(w.v_off[dt]));
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4 * G; ++i) w.pB[i] = 0u;   // P(-1) = 0: phase 0's PV MFMAs add nothing
+  start_wave(w, qh, q0, length, 0);
   // ... and the V(-1) operand they read (V ring slot 3, unit 1) is zeroed, so 0 * V = 0.
   reinterpret_cast<uint4*>(smem + kVRing + 3 * kTileBytes + kUnitBytes)[tid] = make_uint4(0, 0, 0, 0);
 
@@ -631,6 +642,177 @@ __global__ __launch_bounds__(kThreads, 2) void attend_tile192_kernel(
   const int bh = logical / q_blocks;
   query_tile(smem, q, k, v, o, length, bh, qblk * kBM192, length, true, heads, o_batch_stride, o_head_stride,
              o_row_stride);
+}
+
+// Halves launch, for grids that leave CUs idle in one round of 192-query tiles: the block's two
+// waves of a SIMD take the same queries (group qg of four) and the two halves of the keys, so a
+// block of 64, 96 or 128 queries keeps both waves of every SIMD busy and its loop is half as
+// long.  A 64-row ring tile holds one 32-key unit of each half, an iteration is one phase; the
+// halves' acc and l add at the end through LDS (no running max: the sums add as they are), each
+// wave finishing 64 of the 128 output columns.  The price is more copies per MFMA, which is why
+// grids that fill the CUs keep the wider tiles.
+constexpr int kHalfDmaSlot[kDmaPerIter] = {1, 5, 9, 13};
+
+template <bool kMask, int G>
+__device__ __forceinline__ void half_iteration(WaveState<G>& w, const Ctx& c, int first, int u, int r, bool odd) {
+  // reads K units u+1, u+2 and V unit u-1; copies K unit u+4 over K unit u, V unit u+2 over u-2
+  const TileCopy kc = plan_copy<32>(c.smem + kKRing + r * kTileBytes, c.kh, first + u + 4, c.cp);
+  const TileCopy vc = plan_copy<32>(c.smem + kVRing + ((r + 2) & 3) * kTileBytes, c.vh, first + u + 2, c.cp);
+  auto hook = [&](int n) {
+#pragma unroll
+    for (int i = 0; i < kDmaPerIter; ++i)
+      if (kHalfDmaSlot[i] == n) {
+        if (i < kDmaPerTensor) issue_copy(kc, i);
+        else issue_copy(vc, i - kDmaPerTensor);
+      }
+  };
+  const uint8_t* k_cur = c.smem + ((r + 1) & 3) * kTileBytes;    // less kKRing, as in iteration
+  const uint8_t* k_next = c.smem + ((r + 2) & 3) * kTileBytes;
+  const uint8_t* v_cur = c.smem + kVRing + ((r + 3) & 3) * kTileBytes;
+  const int key0 = (first + u) * 32;
+  if (odd) phase<kMask, G>(w, w.sB, w.sA, w.pA, w.pB, k_cur, v_cur, k_next, key0, c.length, c.h, hook);
+  else phase<kMask, G>(w, w.sA, w.sB, w.pB, w.pA, k_cur, v_cur, k_next, key0, c.length, c.h, hook);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(kDmaPerIter) : "memory");
+}
+
+// One wave's half of the keys for its 16 G queries from q0, and the sum with its partner's; writes
+// O.  Every wave of the block calls it with the same unit count, so the barriers match.
+template <int G>
+__device__ __forceinline__ void attend_half(uint8_t* smem, const uint16_t* __restrict__ q,
+                                            const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+                                            uint16_t* __restrict__ o, int length, int bh, int q0, int half, int qg,
+                                            int heads, int64_t o_batch_stride, int64_t o_head_stride,
+                                            int64_t o_row_stride) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int units = (length + 31) / 32;   // 32-key units of the sequence
+  const int n = (units + 1) / 2;          // phases; the second half's last unit may lie past the end
+  const int first = half * n;             // this half's first unit (wave / 4 = half: it copies its own keys)
+  Ctx c;
+  c.smem = smem;
+  c.h = lane >> 4;
+  c.length = length;
+  c.cp.last_tile = units - 1;
+  c.cp.lds_wave_off = wave * kRowsPerWave * kRowBytes;
+  const int rows_last = length - (units - 1) * 32;
+#pragma unroll
+  for (int i = 0; i < kDmaPerTensor; ++i) {
+    const int row = (wave & 3) * kRowsPerWave + i * 4 + (lane >> 4);   // within the unit
+    const uint32_t chunk_off = ((lane & 15) ^ swz(row)) << 4;
+    c.cp.voff[i] = (uint32_t)(row * kRowBytes) + chunk_off;
+    c.cp.voff_last[i] = (uint32_t)(min(row, rows_last - 1) * kRowBytes) + chunk_off;
+  }
+  const int64_t head_off = (int64_t)bh * length * kD;
+  c.kh = k + head_off;
+  c.vh = v + head_off;
+  for (int t = 0; t < 4; ++t) copy_tile<32>(smem + kKRing + t * kTileBytes, c.kh, first + t, c.cp);
+  for (int t = 0; t < 2; ++t) copy_tile<32>(smem + kVRing + t * kTileBytes, c.vh, first + t, c.cp);
+  WaveState<G> w;
+  start_wave(w, q + head_off, q0, length, half * kUnitBytes);
+  // V(-1) of both halves (V ring slot 3), multiplied by P(-1) = 0
+  uint4* const v_before = reinterpret_cast<uint4*>(smem + kVRing + 3 * kTileBytes);
+  v_before[tid] = make_uint4(0, 0, 0, 0);
+  v_before[tid + kThreads] = make_uint4(0, 0, 0, 0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {   // S(0)
+    const int st = i >> 1, kt = i & 1;
+    const bf16x8 a = load_operand(w, i, smem, smem);
+#pragma unroll
+    for (int g = 0; g < G; ++g) w.sA[2 * g + kt] = mfma16(a, w.qreg[st][g], st == 0 ? f32x4{} : w.sA[2 * g + kt]);
+  }
+#pragma unroll
+  for (int i = 0; i < kLead; ++i) w.ops[i % kOpRing] = load_operand(w, i, smem + kTileBytes, smem);
+  __syncthreads();   // K unit 0 is read everywhere: the first iteration copies over it
+
+  const int full = max(length / 32 - n, 0);   // phases whose keys are whole units in both halves
+  int u = 0;
+  for (; u + 4 <= full; u += 4) {
+    half_iteration<false, G>(w, c, first, u, 0, false);
+    half_iteration<false, G>(w, c, first, u + 1, 1, true);
+    half_iteration<false, G>(w, c, first, u + 2, 2, false);
+    half_iteration<false, G>(w, c, first, u + 3, 3, true);
+  }
+  for (; u < n; u += 2) {
+    half_iteration<true, G>(w, c, first, u, u & 3, false);
+    if (u + 1 < n) half_iteration<true, G>(w, c, first, u + 1, (u + 1) & 3, true);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  {
+    const uint8_t* v_last = smem + kVRing + ((n - 1) & 3) * kTileBytes;
+    uint32_t p[4 * G];
+#pragma unroll
+    for (int i = 0; i < 4 * G; ++i) p[i] = (n & 1) ? w.pA[i] : w.pB[i];
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) {
+      const bf16x8 a = load_operand(w, 8 + dt, v_last, v_last);
+#pragma unroll
+      for (int g = 0; g < G; ++g) w.oacc[dt][g] = mfma16(a, p_operand<G>(p, g), w.oacc[dt][g]);
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) w.lacc[g] = mfma16(w.ones, p_operand<G>(p, g), w.lacc[g]);
+  }
+  __syncthreads();   // every wave is done with the rings
+
+  // Wave (half, qg) gives d tiles 4 - 4 half .. + 3 and its l, and finishes the other four.
+  const int mine = half * 4 + qg, theirs = (1 - half) * 4 + qg;
+  f32x4* const accs = reinterpret_cast<f32x4*>(smem) + lane;   // 8 waves x 8 fragments
+  float* const ls = reinterpret_cast<float*>(smem + 8 * 8 * 64 * 16);
+  f32x4 sum[4][G];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      accs[(mine * 8 + j * G + g) * 64] = half ? w.oacc[j][g] : w.oacc[4 + j][g];
+      sum[j][g] = half ? w.oacc[4 + j][g] : w.oacc[j][g];
+    }
+  if (lane < 16)
+#pragma unroll
+    for (int g = 0; g < G; ++g) ls[mine * 32 + g * 16 + lane] = w.lacc[g][0];
+  __syncthreads();
+  const int col = lane & 15;
+  const int b = bh / heads, hd = bh - b * heads;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int qi = q0 + g * 16 + col;
+    const float l = ls[qg * 32 + g * 16 + col] + ls[(4 + qg) * 32 + g * 16 + col];
+    if (qi >= length) continue;
+    uint16_t* orow = o + b * o_batch_stride + hd * o_head_stride + (int64_t)qi * o_row_stride;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 acc = sum[j][g] + accs[(theirs * 8 + j * G + g) * 64];
+      const int d0 = (half * 4 + j) * 16 + c.h * 4;
+      uint2 val;
+      val.x = flk::pack_bf16x2(acc[0] / l, acc[1] / l);
+      val.y = flk::pack_bf16x2(acc[2] / l, acc[3] / l);
+      *reinterpret_cast<uint2*>(orow + d0) = val;
+    }
+  }
+}
+
+// kTQ queries per block: 128 (four groups of 32), 64 (four of 16) or 96 (two of each; a SIMD's two
+// waves, w and w + 4, take one of each).
+template <int kTQ>
+__global__ __launch_bounds__(kThreads, 2) void attend_halves_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    uint16_t* __restrict__ o, int length, int q_blocks, int total_blocks, int heads, int64_t o_batch_stride,
+    int64_t o_head_stride, int64_t o_row_stride) {
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kSmemBytes];
+  const int p = blockIdx.x;
+  const int xcd = p % kXcds, local = p / kXcds;
+  const int per = total_blocks / kXcds, extra = total_blocks % kXcds;
+  const int logical = xcd * per + min(xcd, extra) + local;
+  const int qblk = logical % q_blocks, bh = logical / q_blocks;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform branch below
+  const int half = wave >> 2, qg = half ? (wave + 2) & 3 : wave;
+  if (kTQ == 128 || (kTQ == 96 && qg < 2)) {
+    attend_half<2>(smem, q, k, v, o, length, bh, qblk * kTQ + qg * 32, half, qg, heads, o_batch_stride, o_head_stride,
+                   o_row_stride);
+  } else {
+    attend_half<1>(smem, q, k, v, o, length, bh, kTQ == 96 ? qblk * kTQ + 32 + qg * 16 : qblk * kTQ + qg * 16, half,
+                   qg, heads, o_batch_stride, o_head_stride, o_row_stride);
+  }
 }
 
 // Rounds launch, for grids of more than one round: each XCD takes a contiguous range of the
@@ -1088,6 +1270,34 @@ extern "C" int flk_attend_balanced_to(const void* q, const void* k, const void* 
   return flk_launch_status();
 }
 
+namespace {
+
+int64_t half_tiles(int length, int queries) { return ((int64_t)length + queries - 1) / queries; }
+
+}  // namespace
+
+extern "C" int flk_attend_halves_to(const void* q, const void* k, const void* v, void* o, int batch, int heads,
+                                    int length, int head_dim, int64_t o_batch_stride, int64_t o_head_stride,
+                                    int64_t o_row_stride, int queries, void* stream) {
+  const int st = check_attend(q, k, v, o, batch, heads, length, head_dim, o_batch_stride, o_head_stride,
+                              o_row_stride);
+  if (st != FLK_OK) return st == kNothing ? FLK_OK : st;
+  if (queries != 64 && queries != 96 && queries != 128) return FLK_E_INVALID;
+  const int64_t total = half_tiles(length, queries) * batch * heads;
+  if (total > INT32_MAX) return FLK_E_INVALID;
+#define FLK_HALVES(TQ)                                                                                              \
+  hipLaunchKernelGGL(attend_halves_kernel<TQ>, dim3((unsigned)total), dim3(kThreads), 0,                            \
+                     static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(q),                             \
+                     static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), static_cast<uint16_t*>(o),   \
+                     length, (int)half_tiles(length, queries), (int)total, heads, o_batch_stride, o_head_stride,    \
+                     o_row_stride)
+  if (queries == 64) FLK_HALVES(64);
+  else if (queries == 96) FLK_HALVES(96);
+  else FLK_HALVES(128);
+#undef FLK_HALVES
+  return flk_launch_status();
+}
+
 extern "C" int flk_attend_plan(int batch, int heads, int length, int* splits, int64_t* workspace_bytes) {
   if (batch < 0 || heads < 0 || length < 0 || !splits || !workspace_bytes) return FLK_E_INVALID;
   int s = 1;
@@ -1099,6 +1309,32 @@ extern "C" int flk_attend_plan(int batch, int heads, int length, int* splits, in
   }
   *splits = s;
   *workspace_bytes = s > 1 ? split_workspace_bytes(batch, heads, length, s) : 0;
+  return FLK_OK;
+}
+
+// The halves launch of a shape: the smallest block of 64, 96 or 128 queries that fits the CUs in one
+// round, unless the key split is faster.  Estimates in ns, fitted to measured launches: a halves
+// block takes 8.4 / 10 / 12 a key and 5 us around them, a split range 17 a key, its partials and
+// the merge 9 us and 60 ns a block.  Measured (us; heads x tokens, halves against the launch it
+// replaces): 24 x 768 15.5 / 20.7, 24 x 1280 26.2 / 31.9, 12 x 1536 22.7 / 28.8, 6 x 2048 23.0 /
+// 26.1, 5 x 4608 55.7 / 62.4, 1 x 1024 13.2 / 18.5; where the split stays: 3 x 4608 44.5 / 43.4,
+// 1 x 4608 40.5 / 26.4, 3 x 8192 109 / 100.  24 x 1536 (288 blocks of 128) keeps 192-query tiles.
+extern "C" int flk_attend_halves_plan(int batch, int heads, int length, int* queries) {
+  if (batch < 0 || heads < 0 || length < 0 || !queries) return FLK_E_INVALID;
+  *queries = 0;
+  const int64_t bh = (int64_t)batch * heads;
+  if (bh == 0 || length == 0 || bh > kCUs) return FLK_OK;
+  int tq = 0, ns_per_key = 0;
+  if (half_tiles(length, 64) * bh <= kCUs) tq = 64, ns_per_key = 84;
+  else if (half_tiles(length, 96) * bh <= kCUs) tq = 96, ns_per_key = 100;
+  else if (half_tiles(length, 128) * bh <= kCUs) tq = 128, ns_per_key = 120;
+  else return FLK_OK;
+  int splits = 1;
+  int64_t bytes = 0;
+  flk_attend_plan(batch, heads, length, &splits, &bytes);
+  const int64_t halves_ns = 5000 + (int64_t)length * ns_per_key / 10;
+  const int64_t split_ns = 9000 + 17 * (int64_t)length / splits + 60 * splits * q_tiles(length) * bh;
+  if (splits == 1 || halves_ns < split_ns) *queries = tq;
   return FLK_OK;
 }
 

@@ -287,9 +287,9 @@ def attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, block: int | No
     """kernels.py:105-145 -- bounded flash attention (no running max), q pre-scaled by
     1/sqrt(D).  q, k, v (B, H, L, D) bf16 -> o (B, H, L, D) bf16.
 
-    Grids too small to fill the GPU (few heads or short sequences) cut the keys into ranges
-    whose partial sums are added afterwards (flk_attend_split_to); ``splits`` overrides the
-    automatic choice (1 = never split)."""
+    Grids too small to fill the GPU (few heads or short sequences) cut the keys in two inside
+    each block (flk_attend_halves_to) or into ranges whose partial sums are added afterwards
+    (flk_attend_split_to); ``splits`` overrides the automatic choice (1 = never cut)."""
     if interpret:
         raise ValueError("interpret=True is Pallas' CPU emulation; flicker_amd has one HIP path")
     for name, t in (("q", q), ("k", k), ("v", v)):
@@ -350,6 +350,8 @@ def attend_merged(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
 def attend_kernels(batch: int, heads: int, length: int) -> tuple[str, ...]:
     """Names of the kernels ``attend`` launches for a (batch, heads, length, 128) problem, in
     order, as kernel traces show them (for profiling; the choice is _launch_attend's)."""
+    if _lib.attend_halves_plan(batch, heads, length):
+        return ("attend_halves_kernel",)
     splits, _ = _lib.attend_plan(batch, heads, length)
     if splits > 1:
         return ("attend_kernel<true>", "attend_merge_kernel")
@@ -359,15 +361,21 @@ def attend_kernels(batch: int, heads: int, length: int) -> tuple[str, ...]:
 
 
 def _launch_attend(q, k, v, out, o_strides, splits: int | None, balanced: bool | None = None) -> None:
-    """O through strides (batch, head, row): with ``splits`` None the plan's choice -- the
-    key-split path when the grid is small, the balanced path (flk_attend_balanced_to: one
-    persistent block per CU, the last round's tiles cut by keys) when flk_attend_balanced_plan
-    prefers it, else one block per tile.  An explicit ``splits`` forces that split count
-    (1 = one block per tile, flk_attend_to); ``balanced=True`` forces the balanced launch."""
+    """O through strides (batch, head, row): with ``splits`` None the plan's choice -- the halves
+    path (flk_attend_halves_to: small blocks whose waves cut the keys in two) or the key-split
+    path when the grid is small, the balanced path (flk_attend_balanced_to: one persistent block
+    per CU, the last round's tiles cut by keys) when flk_attend_balanced_plan prefers it, else
+    one block per tile.  An explicit ``splits`` forces that split count (1 = one block per tile,
+    flk_attend_to); ``balanced=True`` forces the balanced launch."""
     batch, heads, length, dim = q.shape
+    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), batch, heads, length, dim, *o_strides)
+    if splits is None and balanced is None:
+        queries = _lib.attend_halves_plan(batch, heads, length)
+        if queries:
+            _lib.run("flk_attend_halves_to", (q, k, v, out), *args, queries, _lib.stream_of(q))
+            return
     planned, _ = _lib.attend_plan(batch, heads, length)
     groups = max(1, -(-length // 256))
-    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), batch, heads, length, dim, *o_strides)
     if balanced is None:
         balanced = splits is None and planned == 1 and _lib.attend_balanced_plan(batch, heads, length)[0] > 0
     if balanced:

@@ -238,6 +238,18 @@ int flk_attend_balanced_plan(int batch, int heads, int length, int* grid, int64_
                              int64_t* counters_offset);
 
 /*
+ * flk_attend_to with blocks of `queries` = 64, 96 or 128 queries whose waves also cut the keys in
+ * two, the halves' sums added on chip: for grids that leave CUs idle in one round of 192-query
+ * tiles.  The result differs from flk_attend's in float32 summation order only, and depends on
+ * the shape alone.  flk_attend_halves_plan gives the choice for a shape: the smallest of the
+ * three whose blocks fit the CUs in one round, or 0 where another launch is faster.
+ */
+int flk_attend_halves_plan(int batch, int heads, int length, int* queries);
+int flk_attend_halves_to(const void* q, const void* k, const void* v, void* o, int batch, int heads,
+                         int length, int head_dim, int64_t o_batch_stride, int64_t o_head_stride,
+                         int64_t o_row_stride, int queries, void* stream);
+
+/*
  * The split count flk_attend_split_to should use for a shape, and its workspace size.
  * *splits = 1 (workspace 0) when the plain grid already has >= 192 blocks of 256 queries.
  * Otherwise it takes as many ranges as fill the 256 CUs once, keeping at least 512 keys per

@@ -310,3 +310,38 @@ def test_attend_key_split_random_small_grids(device):
         assert np.mean(diff > 0) <= 0.01, label
         if length <= 1200:
             tight_gate(label, got, P.attend_bounded(to_np(q), to_np(k), to_np(v)))
+
+
+@pytest.mark.parametrize("queries", [64, 96, 128])
+@pytest.mark.parametrize("length", [1, 31, 32, 33, 65, 97, 127, 192, 289, 320, 351, 640, 1001])
+def test_attend_halves_matches_oracle(device, queries, length):
+    """flk_attend_halves_to with each block size: a second half that is empty, one unit shorter or
+    ends in a partial unit, fewer phases than the unrolled loop, blocks that are not full.  The
+    same gate as the one-pass kernel and within rounding of it (another f32 summation order), rows
+    past the end untouched."""
+    q, k, v = prepped_case(1, 2, length, seed=length)
+    d = [t.to(device) for t in (q, k, v)]
+    out = torch.full((1, 2, length + 3, D), 7.0, dtype=torch.bfloat16, device=device)
+    _lib.run("flk_attend_halves_to", (*d, out), *(t.data_ptr() for t in d), out.data_ptr(), 1, 2, length, D,
+             2 * (length + 3) * D, (length + 3) * D, D, queries, _lib.stream_of(out))
+    torch.cuda.synchronize()
+    assert bool((out[:, :, length:] == 7.0).all())
+    got = to_np(out[:, :, :length].contiguous())
+    tight_gate(f"halves {queries} L{length}", got, P.attend_bounded(to_np(q), to_np(k), to_np(v)))
+    one = run_attend(q, k, v, device, 1)
+    diff = np.abs(got.astype(np.float64) - one)
+    assert np.all(diff <= 2 * np.abs(one) * 2.0 ** -8 + 1e-6)   # one bf16 ulp of either value
+    assert np.mean(diff > 0) <= 0.01
+
+
+@pytest.mark.parametrize("batch,heads,length", [(1, 24, 768), (1, 24, 640), (2, 6, 1300), (1, 3, 700)])
+def test_attend_takes_halves(device, batch, heads, length):
+    """The automatic choice takes the halves launch, merged and head-major, every head the same."""
+    assert kernels.attend_kernels(batch, heads, length) == ("attend_halves_kernel",)
+    q, k, v = (t.to(device) for t in prepped_case(batch, heads, length, seed=heads + length))
+    got = kernels.attend_merged(q, k, v)
+    one = kernels.attend_merged(q, k, v, splits=1)
+    torch.cuda.synchronize()
+    diff = np.abs(to_np(got).astype(np.float64) - to_np(one))
+    assert np.all(diff <= 2 * np.abs(to_np(one)) * 2.0 ** -8 + 1e-6)
+    assert np.mean(diff > 0) <= 0.01

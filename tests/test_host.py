@@ -103,6 +103,22 @@ def test_attend_split_plan_and_validation(lib):
                    "flk_attend_plan")
 
 
+def test_attend_halves_plan_and_validation(lib):
+    """flk_attend_halves_plan: the smallest block whose grid fits 256 CUs, none where the grid does
+    not fit or the key split is faster; flk_attend_halves_to refuses other block sizes."""
+    cases = {(1, 24, 640): 64, (1, 24, 641): 96, (1, 24, 960): 96, (1, 24, 961): 128, (1, 24, 1280): 128,
+             (1, 24, 1281): 0, (1, 24, 4608): 0, (1, 3, 4608): 0, (1, 1, 4608): 0, (1, 5, 4608): 96, (1, 6, 2048): 64,
+             (1, 1, 1): 64, (1, 256, 64): 64, (1, 257, 64): 0, (0, 3, 64): 0, (1, 2, 2 ** 31 - 257): 0}
+    for shape, want in cases.items():
+        assert _lib.attend_halves_plan(*shape) == want, (shape, _lib.attend_halves_plan(*shape))
+    f = lib.flk_attend_halves_to
+    args = (FAKE, FAKE, FAKE, FAKE, 1, 24, 768, 128, 768 * 3072, 128, 3072)
+    assert f(*args, 192, None) == _lib.FLK_E_INVALID
+    assert f(*args, 0, None) == _lib.FLK_E_INVALID
+    assert f(FAKE, FAKE, FAKE, FAKE + 4, *args[4:], 64, None) == _lib.FLK_E_ALIGN
+    assert f(FAKE, FAKE, FAKE, FAKE, 0, *args[5:], 64, None) == _lib.FLK_OK   # empty
+
+
 def test_attend_balanced_plan_and_validation(lib):
     """flk_attend_balanced_plan prefers the balanced launch only where every XCD has a full
     round of 32 tiles, at most 16 are left over on the fullest XCD, and each CU's share of
