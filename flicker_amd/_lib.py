@@ -105,7 +105,7 @@ def check(status: int, what: str) -> None:
 def stream_of(t: torch.Tensor) -> int:
     """Raw hipStream_t of torch's current stream on the tensor's device (the integer handle,
     without building a torch Stream object per call)."""
-    return torch._C._cuda_getCurrentRawStream(t.device.index)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def device_of(*tensors) -> torch.device:
@@ -121,14 +121,24 @@ def device_of(*tensors) -> torch.device:
 
 def run(name: str, tensors, *args) -> None:
     """Call entry point ``name`` with the tensors' GPU current -- a HIP launch goes to the
-    current device, whatever device the tensors live on -- and raise on a non-zero status."""
-    device = device_of(*tensors)
+    current device, whatever device the tensors live on -- and raise on a non-zero status.
+    Small launches are bound by this path, so the common case compares device indices (no
+    device objects) and leaves the error reports to device_of and check."""
+    index = tensors[0].get_device()
+    for t in tensors:
+        if t is not None and t.get_device() != index:
+            index = -1
+            break
+    if index < 0:
+        index = device_of(*tensors).index
     fn = getattr(lib(), name)
-    if torch.cuda.current_device() == device.index:
-        check(fn(*args), name)
-        return
-    with torch.cuda.device(device):
-        check(fn(*args), name)
+    if torch._C._cuda_getDevice() == index:
+        status = fn(*args)
+    else:
+        with torch.cuda.device(index):
+            status = fn(*args)
+    if status != FLK_OK:
+        check(status, name)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

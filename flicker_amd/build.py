@@ -1,4 +1,4 @@
-"""Build recipe for libflicker_hip.so (hipcc, gfx950 only).
+"""Build recipe for libflicker_hip.so (hipcc, gfx950 only) and _native.so (g++, host only).
 
 Every ``csrc/*.hip`` file is compiled to an object in parallel, then linked into
 ``flicker_amd/libflicker_hip.so`` next to this file, so the library travels with
@@ -20,6 +20,7 @@ CSRC = PKG / "csrc"
 INCLUDE = ROOT / "include"
 BUILD = PKG / "_build"
 LIB = PKG / "libflicker_hip.so"
+NATIVE = PKG / "_native.so"
 ARCH = "gfx950"
 
 # Packed float32 VALU ops are turned off for all device code; -O3 would otherwise form them.
@@ -64,7 +65,27 @@ def build(verbose: bool = False, jobs: int | None = None) -> pathlib.Path:
     tmp = LIB.with_suffix(".so.tmp")
     _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)], verbose)
     os.replace(tmp, LIB)
+    build_native(verbose)
     return LIB
+
+
+def build_native(verbose: bool = False) -> pathlib.Path:
+    """Compile the host-only Python module over libflicker_hip.so (the hot entry points' per-call
+    path) against this interpreter and its torch; returns its path."""
+    import sysconfig
+
+    import torch
+    torch_dir = pathlib.Path(torch.__file__).resolve().parent
+    includes = [INCLUDE, torch_dir / "include", torch_dir / "include/torch/csrc/api/include",
+                pathlib.Path(hipcc()).resolve().parent.parent / "include", sysconfig.get_paths()["include"]]
+    tmp = NATIVE.with_suffix(".so.tmp")
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+          "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          f"-I{includes[0]}", *(f"-isystem{p}" for p in includes[1:]), str(PKG / "csrc_host/native.cpp"), "-o",
+          str(tmp), f"-L{torch_dir / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip",
+          f"-L{PKG}", "-l:libflicker_hip.so", "-Wl,-rpath,$ORIGIN"], verbose)
+    os.replace(tmp, NATIVE)
+    return NATIVE
 
 
 if __name__ == "__main__":

@@ -26,6 +26,11 @@ import torch
 
 from . import _lib
 
+try:
+    from . import _native   # the per-call path of plain operands; returns None for any other call
+except ImportError:         # not built for this interpreter: every call takes the Python path below
+    _native = None
+
 HEAD_DIM = 128  # the only head width the HIP kernels are built for (Klein 4B: 3072 / 24)
 
 
@@ -62,6 +67,8 @@ def row_tile(length: int) -> int | None:
 
 
 def _on_gpu(name: str, t: torch.Tensor) -> None:
+    if isinstance(t, torch.Tensor) and t.is_cuda:
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor, got {type(t).__name__}")
     if t.device.type != "cuda":
@@ -71,8 +78,18 @@ def _on_gpu(name: str, t: torch.Tensor) -> None:
 def _dense_rows(t: torch.Tensor) -> torch.Tensor:
     """Keep a view whose last axis is contiguous and whose other strides keep 16-byte rows;
     anything else is compacted on the device first."""
-    ok = t.stride(-1) == 1 and all(s % 8 == 0 for s in t.stride()[:-1]) and t.data_ptr() % 16 == 0
-    return t if ok else t.contiguous()
+    if t.data_ptr() % 16:
+        return t.contiguous()
+    *outer, inner = t.stride()
+    for s in outer:
+        if s % 8:
+            return t.contiguous()
+    return t if inner == 1 else t.contiguous()
+
+
+def _vector(t: torch.Tensor) -> torch.Tensor:
+    """``t`` as a contiguous 1-D tensor, itself where it is one."""
+    return t if t.dim() == 1 and t.is_contiguous() else t.reshape(-1).contiguous()
 
 
 def lane_pair(freqs: torch.Tensor, q_gain: float = 1.0) -> Freqs:
@@ -95,12 +112,16 @@ def lane_pair(freqs: torch.Tensor, q_gain: float = 1.0) -> Freqs:
 
 def _table_args(freqs: Freqs, length: int, head_dim: int):
     cos, sin, _ = freqs
-    for name, t in (("freqs.cos", cos), ("freqs.sin", sin)):
-        _on_gpu(name, t)
-    if cos.shape != (length, head_dim) or sin.shape != (length, head_dim):
+    _on_gpu("freqs.cos", cos)
+    _on_gpu("freqs.sin", sin)
+    shape = (length, head_dim)
+    if cos.shape != shape or sin.shape != shape:
         raise ValueError(f"freqs tables must be ({length}, {head_dim}), got {tuple(cos.shape)} / {tuple(sin.shape)}")
     if cos.dtype != torch.float32 or sin.dtype != torch.float32:
         raise TypeError("freqs.cos / freqs.sin must be float32")
+    dense = (head_dim, 1)
+    if cos.stride() == dense and sin.stride() == dense and not (cos.data_ptr() | sin.data_ptr()) & 15:
+        return cos, sin   # the tables as rope_lanes and lane_pair make them
     cos = cos if cos.stride(1) == 1 and cos.stride(0) % 4 == 0 and cos.data_ptr() % 16 == 0 else cos.contiguous()
     sin = sin if sin.stride(1) == 1 and sin.stride(0) % 4 == 0 and sin.data_ptr() % 16 == 0 else sin.contiguous()
     if sin.stride(0) != cos.stride(0):
@@ -140,8 +161,8 @@ def _qk_operands(qkv, q_scale, k_scale, freqs, num_heads: int, qk_f32: bool = Fa
         rope = _table_args(freqs, length, head_dim)
     else:
         raise TypeError(f"freqs must be Freqs or PositionIds, got {type(freqs).__name__}")
-    for name, t in (("q_scale", q_scale), ("k_scale", k_scale)):
-        _on_gpu(name, t)
+    _on_gpu("q_scale", q_scale)
+    _on_gpu("k_scale", k_scale)
     if q_scale.numel() != head_dim or k_scale.numel() != head_dim:
         raise ValueError(f"q_scale / k_scale must hold {head_dim} values")
     if q_scale.dtype != k_scale.dtype or q_scale.dtype not in (torch.bfloat16, torch.float32):
@@ -149,8 +170,7 @@ def _qk_operands(qkv, q_scale, k_scale, freqs, num_heads: int, qk_f32: bool = Fa
     if qk_f32 and (q_scale.dtype != torch.float32 or isinstance(freqs, PositionIds) or freqs.q_gain != 1.0):
         raise ValueError("float32 q / k outputs are the plain branch's: float32 scales, lane tables, gain 1")
     qkv = _dense_rows(qkv)
-    q_scale = q_scale.reshape(-1).contiguous()
-    k_scale = k_scale.reshape(-1).contiguous()
+    q_scale, k_scale = _vector(q_scale), _vector(k_scale)
     return qkv, q_scale, k_scale, freqs, rope, head_dim
 
 
@@ -169,6 +189,10 @@ def _launch_qk_prep(qkv, q_scale, k_scale, freqs, num_heads: int, out, out_offse
     """qk_prep's launch.  ``qk_f32``: the plain branch of qkv_prep with float32 scales
     (modules.py:78-80, where rms_norm's product and apply_rope's result stay float32): q and
     k come out float32, unrounded and without a query gain (flk_qk_prep_f32); v stays bf16."""
+    if _native is not None and out is None and not qk_f32 and out_offset == 0 and type(freqs) is Freqs:
+        done = _native.qk_prep(qkv, q_scale, k_scale, freqs.cos, freqs.sin, freqs.q_gain, num_heads)
+        if done is not None:
+            return done
     batch, length, _ = qkv.shape
     qkv, q_scale, k_scale, freqs, rope, head_dim = _qk_operands(qkv, q_scale, k_scale, freqs, num_heads, qk_f32)
     q_gain = freqs.q_gain
@@ -176,8 +200,9 @@ def _launch_qk_prep(qkv, q_scale, k_scale, freqs, num_heads: int, out, out_offse
     if out is None:
         if out_offset:
             raise ValueError("out_offset needs out=(q, k, v)")
-        shape = (batch, num_heads, length, head_dim)
-        out = tuple(torch.empty(shape, dtype=dt, device=qkv.device) for dt in (qk_dtype, qk_dtype, torch.bfloat16))
+        shape, device = (batch, num_heads, length, head_dim), qkv.device
+        out = (torch.empty(shape, dtype=qk_dtype, device=device), torch.empty(shape, dtype=qk_dtype, device=device),
+               torch.empty(shape, dtype=torch.bfloat16, device=device))
         out_length = length
     else:
         out = tuple(out)
@@ -206,8 +231,7 @@ def _launch_qk_prep(qkv, q_scale, k_scale, freqs, num_heads: int, out, out_offse
     else:
         cos, sin = rope
         _lib.run("flk_qk_prep", (qkv, cos, sin, q_scale, k_scale, *out),
-                 qkv.data_ptr(), qkv.stride(0), qkv.stride(1), cos.data_ptr(), sin.data_ptr(), cos.stride(0),
-                 *common)
+                 qkv.data_ptr(), *qkv.stride()[:2], cos.data_ptr(), sin.data_ptr(), cos.stride(0), *common)
     return out
 
 
@@ -308,6 +332,10 @@ def attend_merged(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
     kernel: the attention epilogue writes o[b, t, h*D:(h+1)*D] directly, so the transposing
     copy of merge_heads disappears.  q, k, v (B, H, L, D) bf16 -> (B, L, H*D) bf16; ``out`` may
     be a (B, L, H*D) view whose rows are strided (e.g. columns of a wider buffer)."""
+    if _native is not None and out is None and splits is None:
+        done = _native.attend_merged(q, k, v)
+        if done is not None:
+            return done
     for name, t in (("q", q), ("k", k), ("v", v)):
         if t.dim() != 4:
             raise ValueError(f"{name} must be (B, H, L, D), got {tuple(t.shape)}")

@@ -12,7 +12,8 @@ from __future__ import annotations
 
 import torch
 
-from .kernels import Freqs, PositionIds, _launch_qk_prep, _launch_qk_prep_pair, attend_merged, lane_pair, row_tile
+from .kernels import (Freqs, PositionIds, _launch_qk_prep, _launch_qk_prep_pair, _native, attend_merged, lane_pair,
+                      row_tile)
 
 
 def heads(qkv: torch.Tensor, num_heads: int):
@@ -84,6 +85,12 @@ def double_attention(txt_qkv, img_qkv, txt_scales, img_scales, freqs: Freqs | Po
     they are read only by a stream whose length has no row tile (the gate's plain branch)."""
     batch, num_txt, width = txt_qkv.shape
     num_img = img_qkv.shape[1]
+    fused = type(freqs) is Freqs and row_tile(num_txt) is not None and row_tile(num_img) is not None
+    if _native is not None and fused:
+        done = _native.double_attention(txt_qkv, *txt_scales, img_qkv, *img_scales, freqs.cos, freqs.sin,
+                                        freqs.q_gain, num_heads)
+        if done is not None:
+            return done
     for name, length, scales in (("text", num_txt, txt_scales), ("image", num_img, img_scales)):
         if row_tile(length) is None and scales[0].dtype == torch.float32:
             raise TypeError(f"double_attention: the {name} stream (L={length}, no row tile) takes qkv_prep's plain "
@@ -91,8 +98,7 @@ def double_attention(txt_qkv, img_qkv, txt_scales, img_scales, freqs: Freqs | Po
     head_dim = width // (3 * num_heads)
     shape = (batch, num_heads, num_txt + num_img, head_dim)
     joint = tuple(torch.empty(shape, dtype=torch.bfloat16, device=txt_qkv.device) for _ in range(3))
-    if (isinstance(freqs, Freqs) and row_tile(num_txt) is not None and row_tile(num_img) is not None
-            and txt_scales[0].dtype == img_scales[0].dtype and img_qkv.shape[0] == batch):
+    if fused and txt_scales[0].dtype == img_scales[0].dtype and img_qkv.shape[0] == batch:
         _launch_qk_prep_pair((txt_qkv, *txt_scales, _slice(freqs, 0, num_txt)),
                              (img_qkv, *img_scales, _slice(freqs, num_txt, num_txt + num_img)), num_heads, joint)
     else:

@@ -25,7 +25,7 @@ from typing import NamedTuple
 import torch
 
 from . import _lib
-from .kernels import _on_gpu
+from .kernels import _native, _on_gpu, _vector
 
 
 class QuantizedLinear(NamedTuple):
@@ -63,6 +63,8 @@ def _f32(name: str, t: torch.Tensor, n: int, device) -> torch.Tensor:
     _on_gpu(name, t)
     if t.shape != (n,):
         raise ValueError(f"{name} must have shape ({n},), got {tuple(t.shape)}")
+    if t.dtype == torch.float32 and t.device == device and t.is_contiguous():
+        return t
     return t.to(device=device, dtype=torch.float32).contiguous()
 
 
@@ -226,10 +228,13 @@ def gemm(xq: torch.Tensor, a_scale: torch.Tensor, wq_t: torch.Tensor, w_scale: t
 
 def linear(x: torch.Tensor, qw: QuantizedLinear, *, out: torch.Tensor | None = None) -> torch.Tensor:
     """int8 stand-in for ``linear(x, w)`` (nn.py:13-14): (..., K) bf16 -> (..., N) bf16."""
-    lead = x.shape[:-1]
+    if _native is not None and out is None:
+        y = _native.linear(x, qw.wq_t, qw.w_scale, qw.inv_smooth)
+        if y is not None:
+            return y
     xq, a_scale = quantize_act(x, qw.inv_smooth)
     y = gemm(xq, a_scale, qw.wq_t, qw.w_scale, out=None if out is None else out.view(-1, qw.out_features))
-    return y.reshape(*lead, qw.out_features) if out is None else out
+    return y.view(*x.shape[:-1], qw.out_features) if out is None else out
 
 
 def _qk_stream(x, qw: QuantizedLinear, q_scale, k_scale, freqs, num_heads: int, modulation, quantized=None):
@@ -258,7 +263,7 @@ def _qk_stream(x, qw: QuantizedLinear, q_scale, k_scale, freqs, num_heads: int, 
     if q_scale.dtype != k_scale.dtype or q_scale.dtype not in (torch.bfloat16, torch.float32) \
             or q_scale.numel() != HEAD_DIM or k_scale.numel() != HEAD_DIM:
         raise ValueError(f"q_scale / k_scale must be {HEAD_DIM} bfloat16 or float32 values of one dtype")
-    q_scale, k_scale = q_scale.reshape(-1).contiguous(), k_scale.reshape(-1).contiguous()
+    q_scale, k_scale = _vector(q_scale), _vector(k_scale)
     if quantized is not None:
         xq, a_scale = quantized
     elif modulation is None:
