@@ -141,6 +141,25 @@ def run(name: str, tensors, *args) -> None:
         check(status, name)
 
 
+class _Native:
+    """The functions of the native per-call path (csrc_host/native.cpp), bound at first use: importing
+    this package loads no library, so a build can replace both.  Where the module is not built
+    for this interpreter each function returns None, and every call takes its Python path."""
+
+    def __getattr__(self, name: str):
+        try:
+            from . import _native
+            fn = getattr(_native, name)
+        except ImportError:
+            def fn(*_):
+                return None
+        setattr(self, name, fn)
+        return fn
+
+
+native = _Native()
+
+
 def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 

@@ -26,10 +26,7 @@ import torch
 
 from . import _lib
 
-try:
-    from . import _native   # the per-call path of plain operands; returns None for any other call
-except ImportError:         # not built for this interpreter: every call takes the Python path below
-    _native = None
+_native = _lib.native   # the per-call path of plain operands; returns None for any other call
 
 HEAD_DIM = 128  # the only head width the HIP kernels are built for (Klein 4B: 3072 / 24)
 
