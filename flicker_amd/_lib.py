@@ -44,6 +44,7 @@ SIGNATURES = {
     "flk_absmax_rows": (_i, [_p, _i64, _i64, _i64, _p, _p]),
     "flk_absmax_cols": (_i, [_p, _i64, _i64, _i64, _i, _p, _p]),
     "flk_smooth_factors": (_i, [_p, _p, _i64, _p, _p, _p]),
+    "flk_weight_smooth": (_i, [_p, _i64, _i64, _i64, _p, _p, _p, _p]),
     "flk_quantize_weight": (_i, [_p, _i64, _p, _i, _i, _p, _p, _p]),
     "flk_quantize_act": (_i, [_p, _i64, _p, _i, _i, _p, _p, _p]),
     "flk_quantize_act_modulated": (_i, [_p, _i64, _p, _p, _i64, _i, _p, _i, _i, _p, _p, _p, _i64, _p]),

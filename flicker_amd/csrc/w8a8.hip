@@ -117,10 +117,19 @@ __device__ __forceinline__ void unpack_bf16x8(const uint4& r, float (&f)[8]) {
 
 // ---------------------------------------------------------------- calibration ----------
 
+// s = sqrt(xa) / sqrt(wa) (1 where either maximum is 0).
+__device__ __forceinline__ float smooth_factor(float xa, float wa) {
+  return xa > 0.0f && wa > 0.0f ? __builtin_sqrtf(xa) / __builtin_sqrtf(wa) : 1.0f;
+}
+
 // out[r] = max_c |x[r, c]|; one wave per row, 8 columns per lane step (cols % 8 == 0).
+// kSmooth: out holds the smoothing factors of the row maxima and xa instead, and inv their inverses
+// (a weight's rows are its input channels): one launch less before a weight's quantisation.
+template <bool kSmooth>
 __global__ __launch_bounds__(256) void absmax_rows_kernel(const uint16_t* __restrict__ x, int64_t rows,
                                                           int64_t cols, int64_t stride,
-                                                          float* __restrict__ out) {
+                                                          float* __restrict__ out, const float* __restrict__ xa,
+                                                          float* __restrict__ inv) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + wave;
   if (row >= rows) return;
@@ -133,7 +142,13 @@ __global__ __launch_bounds__(256) void absmax_rows_kernel(const uint16_t* __rest
     for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(f[i]));
   }
   m = wave_max(m);
-  if (lane == 0) out[row] = m;
+  if (lane == 0) {
+    if constexpr (kSmooth) {
+      m = smooth_factor(xa[row], m);
+      inv[row] = 1.0f / m;
+    }
+    out[row] = m;
+  }
 }
 
 // The start of a column maximum: 0, or the running maximum that is accumulated into (a NaN or a
@@ -202,13 +217,11 @@ __global__ __launch_bounds__(256) void absmax_cols_kernel(const uint16_t* __rest
   if (threadIdx.x < 128 && c < cols && v > 0.0f) atomicMax(reinterpret_cast<int*>(out) + c, __float_as_int(v));
 }
 
-// s = sqrt(xa) / sqrt(wa) (1 where either maximum is 0), inv_s = 1 / s.
 __global__ void smooth_factors_kernel(const float* __restrict__ xa, const float* __restrict__ wa, int64_t k,
                                       float* __restrict__ s, float* __restrict__ inv_s) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= k) return;
-  const float a = xa[i], b = wa[i];
-  const float v = (a > 0.0f && b > 0.0f) ? __builtin_sqrtf(a) / __builtin_sqrtf(b) : 1.0f;
+  const float v = smooth_factor(xa[i], wa[i]);
   s[i] = v;
   inv_s[i] = 1.0f / v;
 }
@@ -1029,16 +1042,35 @@ int64_t column_rows(int64_t rows, int64_t blocks) {
 
 }  // namespace
 
-extern "C" int flk_absmax_rows(const void* x, int64_t rows, int64_t cols, int64_t row_stride, float* out,
-                               void* stream) {
+namespace {
+
+int check_rows(const void* x, int64_t rows, int64_t cols, int64_t row_stride, const float* out) {
   if (rows < 0 || cols < 0 || row_stride < cols) return FLK_E_INVALID;
   if (rows == 0) return FLK_OK;
   if (!x || !out || cols == 0) return FLK_E_INVALID;
   if (cols % 8 || row_stride % 8 || !flk_host_aligned(x, 16) || !flk_host_aligned(out, 4)) return FLK_E_ALIGN;
-  const int64_t blocks = (rows + 3) / 4;
-  if (blocks > INT32_MAX) return FLK_E_INVALID;
-  hipLaunchKernelGGL(absmax_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream),
-                     static_cast<const uint16_t*>(x), rows, cols, row_stride, out);
+  return (rows + 3) / 4 > INT32_MAX ? FLK_E_INVALID : FLK_OK;
+}
+
+}  // namespace
+
+extern "C" int flk_absmax_rows(const void* x, int64_t rows, int64_t cols, int64_t row_stride, float* out,
+                               void* stream) {
+  const int st = check_rows(x, rows, cols, row_stride, out);
+  if (st != FLK_OK || rows == 0) return st;
+  hipLaunchKernelGGL(absmax_rows_kernel<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, as_stream(stream),
+                     static_cast<const uint16_t*>(x), rows, cols, row_stride, out, nullptr, nullptr);
+  return flk_launch_status();
+}
+
+extern "C" int flk_weight_smooth(const void* w, int64_t k, int64_t n, int64_t w_row_stride, const float* x_absmax,
+                                 float* s, float* inv_s, void* stream) {
+  const int st = check_rows(w, k, n, w_row_stride, s);
+  if (st != FLK_OK || k == 0) return st;
+  if (!x_absmax || !inv_s) return FLK_E_INVALID;
+  if (!flk_host_aligned(x_absmax, 4) || !flk_host_aligned(inv_s, 4)) return FLK_E_ALIGN;
+  hipLaunchKernelGGL(absmax_rows_kernel<true>, dim3((unsigned)((k + 3) / 4)), dim3(256), 0, as_stream(stream),
+                     static_cast<const uint16_t*>(w), k, n, w_row_stride, s, x_absmax, inv_s);
   return flk_launch_status();
 }
 

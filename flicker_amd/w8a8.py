@@ -118,7 +118,14 @@ def quantize_weight(w: torch.Tensor, smooth: torch.Tensor) -> tuple[torch.Tensor
 
 def quantize_linear(w: torch.Tensor, x_absmax: torch.Tensor) -> QuantizedLinear:
     """Offline half: smoothing factors from calibration statistics, then the int8 weight."""
-    s, inv = smooth_factors(x_absmax, absmax_rows(w))
+    w = _rows("w", w)
+    xa = _f32("x_absmax", x_absmax, x_absmax.shape[0], x_absmax.device)
+    if xa.shape[0] != w.shape[0] or xa.device != w.device:
+        s, inv = smooth_factors(x_absmax, absmax_rows(w))   # its errors and conversions
+    else:
+        s, inv = torch.empty_like(xa), torch.empty_like(xa)
+        _lib.run("flk_weight_smooth", (w, xa, s, inv), w.data_ptr(), w.shape[0], w.shape[1], w.stride(0),
+                 xa.data_ptr(), s.data_ptr(), inv.data_ptr(), _lib.stream_of(w))
     wq_t, w_scale = quantize_weight(w, s)
     return QuantizedLinear(wq_t, w_scale, s, inv)
 

@@ -306,6 +306,13 @@ int flk_absmax_cols(const void* x, int64_t rows, int64_t cols, int64_t row_strid
 int flk_smooth_factors(const float* x_absmax, const float* w_absmax, int64_t k, float* s,
                        float* inv_s, void* stream);
 
+/*
+ * flk_absmax_rows of a weight followed by flk_smooth_factors, in one launch: w (k, n) bf16 rows,
+ * x_absmax (k,) the activation maxima -> s, inv_s (k,), the bits of the two calls.
+ */
+int flk_weight_smooth(const void* w, int64_t k, int64_t n, int64_t w_row_stride, const float* x_absmax,
+                      float* s, float* inv_s, void* stream);
+
 /* Weight W (k, n) bf16 (the reference's (in, out) layout) -> wq_t (n, k) int8, stored
  * transposed so GEMM operands are k-contiguous, and w_scale (n,) f32.  k % 64 == 0,
  * n % 8 == 0. */

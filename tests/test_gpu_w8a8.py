@@ -125,6 +125,22 @@ def test_absmax_cols_row_cuts(device, rows, cols):
     np.testing.assert_array_equal(host(run), np.maximum(want, np.nan_to_num(start.numpy().clip(min=0.0))))
 
 
+@pytest.mark.parametrize("k,n", [(64, 8), (192, 520), (4160, 136)])
+def test_quantize_linear_smooth_equals_two_calls(device, k, n):
+    """quantize_linear's one-launch smoothing factors are the bits of absmax_rows and
+    smooth_factors, rows and channels that are all zero included."""
+    g = torch.Generator().manual_seed(k + n)
+    w = (0.02 * torch.randn(k, n, generator=g)).to(torch.bfloat16)
+    w[3] = 0.0
+    xa = torch.rand(k, generator=g) * 4
+    xa[5] = 0.0
+    w, xa = w.to(device), xa.to(device)
+    qw = w8a8.quantize_linear(w, xa)
+    s, inv = w8a8.smooth_factors(xa, w8a8.absmax_rows(w))
+    assert torch.equal(qw.smooth, s) and torch.equal(qw.inv_smooth, inv)
+    assert float(s[3]) == 1.0 and float(s[5]) == 1.0
+
+
 @pytest.mark.parametrize("k,n", [(64, 8), (192, 72), (128, 264), (4096 + 64, 136)])
 def test_quantize_weight_tile_edges(device, k, n):
     """k of half a 128-row tile and of several cuts, n off the 64- and 128-channel blocks; every
