@@ -125,7 +125,7 @@ def test_absmax_cols_row_cuts(device, rows, cols):
     np.testing.assert_array_equal(host(run), np.maximum(want, np.nan_to_num(start.numpy().clip(min=0.0))))
 
 
-@pytest.mark.parametrize("k,n", [(64, 8), (192, 520), (4160, 136)])
+@pytest.mark.parametrize("k,n", [(64, 8), (192, 520), (64, 3072), (64, 3080), (4160, 136)])
 def test_quantize_linear_smooth_equals_two_calls(device, k, n):
     """quantize_linear's one-launch smoothing factors are the bits of absmax_rows and
     smooth_factors, rows and channels that are all zero included."""
@@ -136,7 +136,9 @@ def test_quantize_linear_smooth_equals_two_calls(device, k, n):
     xa[5] = 0.0
     w, xa = w.to(device), xa.to(device)
     qw = w8a8.quantize_linear(w, xa)
-    s, inv = w8a8.smooth_factors(xa, w8a8.absmax_rows(w))
+    rows = w8a8.absmax_rows(w)
+    assert torch.equal(rows, w.float().abs().amax(1))
+    s, inv = w8a8.smooth_factors(xa, rows)
     assert torch.equal(qw.smooth, s) and torch.equal(qw.inv_smooth, inv)
     assert float(s[3]) == 1.0 and float(s[5]) == 1.0
 
