@@ -739,7 +739,9 @@ __device__ __forceinline__ void attend_half(uint8_t* smem, const uint16_t* __res
     if (u + 1 < n) half_iteration<true, G>(w, c, first, u + 1, (u + 1) & 3, true);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  {
+  // With an odd unit count the second half's last unit lies past the end: its P is 0 and its V slot
+  // repeats the sequence's last unit, where 0 * inf would be NaN, so its products are left out.
+  if (first + n <= units) {
     const uint8_t* v_last = smem + kVRing + ((n - 1) & 3) * kTileBytes;
     uint32_t p[4 * G];
 #pragma unroll

@@ -345,3 +345,26 @@ def test_attend_takes_halves(device, batch, heads, length):
     diff = np.abs(to_np(got).astype(np.float64) - to_np(one))
     assert np.all(diff <= 2 * np.abs(to_np(one)) * 2.0 ** -8 + 1e-6)
     assert np.mean(diff > 0) <= 0.01
+
+
+@pytest.mark.parametrize("length", [31, 96, 224, 320, 351, 1001])
+@pytest.mark.parametrize("queries", [64, 96, 128])
+def test_attend_halves_infinite_values(device, queries, length):
+    """An infinite value of a key near the end is that column's output in every row and touches no
+    other column, where the second half's last unit lies past the end (31, 96, 224, 351) as
+    where it does not."""
+    q, k, v = prepped_case(1, 2, length, seed=length)
+    finite = tuple(t.to(device) for t in (q, k, v))
+    v = v.clone()
+    v[0, 0, length - 3, 5] = float("inf")
+    v[0, 1, length - 4, 70] = -float("inf")
+    out = []
+    for d in (finite, (*finite[:2], v.to(device))):
+        o = torch.empty_like(d[0])
+        _lib.run("flk_attend_halves_to", (*d, o), *(t.data_ptr() for t in d), o.data_ptr(), 1, 2, length, D,
+                 2 * length * D, length * D, D, queries, _lib.stream_of(o))
+        out.append(o)
+    want = out[0].clone()
+    want[0, 0, :, 5], want[0, 1, :, 70] = float("inf"), -float("inf")
+    torch.cuda.synchronize()
+    assert torch.equal(out[1].view(torch.int16), want.view(torch.int16))
