@@ -1148,8 +1148,11 @@ namespace {
 
 // Waves that share a row of K elements: two for the hidden widths, so that a row's chain of
 // reductions is half as long and twice the rows' loads are in flight (one wave per row,
-// 4608 x 3072: 13.1 us, modulated 21.2; two: 10.4, 18.4; 512 rows: 5.2 -> 3.5).
-int row_waves(int k) { return k <= 512 ? 1 : k <= 4096 ? 2 : 4; }
+// 4608 x 3072: 13.1 us, modulated 21.2; two: 10.4, 18.4; 512 rows: 5.2 -> 3.5).  A row of at most
+// three chunks a lane is one wave: sharing it only adds the exchange (two waves, then one, us:
+// 4608 x 1024 6.6 / 4.7, 67584 x 1024 62 / 35, modulated 113 / 71; 4608 x 1536 modulated
+// 12.9 / 10.3; 512 x 1032 modulated 5.0 / 5.2 is the most it loses).
+int row_waves(int k) { return k <= 1536 ? 1 : k <= 4096 ? 2 : 4; }
 
 template <bool kModulate>
 int launch_quantize_act(const QuantGroup& g, int64_t blocks, void* stream) {
@@ -1162,8 +1165,9 @@ int launch_quantize_act(const QuantGroup& g, int64_t blocks, void* stream) {
 #define FLK_QA(W, C) \
   if (full) hipLaunchKernelGGL((quantize_act_kernel<W, C, true, kModulate>), grid, block, 0, st, g); \
   else hipLaunchKernelGGL((quantize_act_kernel<W, C, false, kModulate>), grid, block, 0, st, g)
-  if (waves == 1) { FLK_QA(1, 1); }
-  else if (waves == 2 && chunks == 1) { FLK_QA(2, 1); }
+  if (waves == 1 && chunks == 1) { FLK_QA(1, 1); }
+  else if (waves == 1 && chunks == 2) { FLK_QA(1, 2); }
+  else if (waves == 1) { FLK_QA(1, 3); }
   else if (waves == 2 && chunks == 2) { FLK_QA(2, 2); }
   else if (waves == 2 && chunks == 3) { FLK_QA(2, 3); }
   else if (waves == 2) { FLK_QA(2, 4); }

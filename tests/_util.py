@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -33,3 +35,32 @@ def abs_stats(got: np.ndarray, want: np.ndarray) -> dict:
 
 def describe(label: str, stats: dict) -> str:
     return label + " " + " ".join(f"{k}={v:.3g}" for k, v in stats.items())
+
+
+class _KernelNodeParams(ctypes.Structure):
+    """hipKernelNodeParams (hip_runtime_api.h)."""
+    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p),
+                ("grid", ctypes.c_uint * 3), ("params", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+
+def launches(fn) -> list:
+    """The grid (x, y, z) of every kernel that ``fn`` launches, read from a captured graph."""
+    from flicker_amd import _lib
+    hip = _lib.lib()   # its symbols include those of the HIP runtime it is linked to
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        fn()
+    raw, count = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(count)) == 0
+    nodes = (ctypes.c_void_p * max(1, count.value))()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(count)) == 0
+    grids = []
+    for node in nodes[:count.value]:
+        kind, p = ctypes.c_int(-1), _KernelNodeParams()
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
+        if kind.value == 0:   # hipGraphNodeTypeKernel
+            assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+            grids.append(tuple(p.grid))
+    return grids

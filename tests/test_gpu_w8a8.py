@@ -13,6 +13,8 @@ from flicker_amd import w8a8, workloads
 from oracle import w8a8 as Q
 from oracle.numerics import bf16_bits, from_bf16_bits
 
+from ._util import launches
+
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
 
@@ -456,7 +458,7 @@ def test_modulated_activation_bit_exact(device, batch, length, k):
     assert torch.equal(xq2, xq) and torch.equal(a2, a_scale)
 
 
-@pytest.mark.parametrize("k", [8, 504, 512, 520, 1024, 1032, 2048, 3072, 3080, 4096, 4104, 6144, 6152, 8192])
+@pytest.mark.parametrize("k", [8, 504, 512, 520, 1024, 1032, 1536, 1544, 2048, 3072, 3080, 4096, 4104, 6144, 6152, 8192])
 def test_quantize_act_widths(device, k):
     """Each split of a row over waves and chunks, full and ragged, with a last block that is not
     full; rows of zeros, of values whose scale is subnormal (1 / a overflows) or small, and of
@@ -485,6 +487,19 @@ def test_quantize_act_widths(device, k):
     want_q, want_a = Q.quantize_act(want.reshape(-1, k), inv)
     np.testing.assert_array_equal(host(mq), want_q)
     np.testing.assert_array_equal(host(ma), want_a)
+
+
+@pytest.mark.parametrize("k,rows_per_block", [(512, 4), (520, 4), (1024, 4), (1032, 4), (1536, 4), (1544, 2),
+                                              (4096, 2), (4104, 1)])
+def test_quantize_act_rows_per_block(device, k, rows_per_block):
+    """One wave per row up to 1536 channels, two up to 4096, four past that: more waves of fewer
+    chunks cost rows of 1024 channels up to half as much again."""
+    x = torch.randn(1, 16, k).to(torch.bfloat16).to(device)
+    mod = torch.zeros(1, k, dtype=torch.bfloat16, device=device)
+    inv = torch.ones(k, device=device)
+    want = [(16 // rows_per_block, 1, 1)]
+    assert launches(lambda: w8a8.quantize_act(x, inv)) == want
+    assert launches(lambda: w8a8.quantize_act_modulated(x, mod, mod, inv)) == want
 
 
 def test_modulated_projection_qk_prep(device):
