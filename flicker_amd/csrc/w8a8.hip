@@ -164,8 +164,8 @@ __global__ __launch_bounds__(256) void absmax_rows_kernel(const uint16_t* __rest
   }
 }
 
-// The start of a column maximum: 0, or the running maximum that is accumulated into (a NaN or a
-// negative value there counts as 0, as fmaxf against the first |x| does).
+// The start of a merged column maximum: 0, or the running maximum that is accumulated into (a NaN
+// or a negative value there counts as 0, as fmaxf against the first |x| does).
 __global__ __launch_bounds__(256) void absmax_init_kernel(int64_t cols, int accumulate, float* __restrict__ out) {
   const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (c < cols) out[c] = accumulate ? fmaxf(out[c], 0.0f) : 0.0f;
@@ -215,19 +215,26 @@ __device__ __forceinline__ float column_absmax(float (&red)[16][129], const uint
   return v;
 }
 
-// out[c] = max(out[c], max_r |x[r, c]|), out set by absmax_init_kernel.  HBM-bound: the rows are
-// cut over blockIdx.y so that the pass fills the chip (one block per 128 columns alone was 24
-// blocks at 3072 channels, each a serial walk of the rows).  Block maxima are finite or +inf and
-// never negative, so their int bits order as the floats do and an integer atomic merges them.
-// 4608 x 3072 (28 MB): 6.5 us + 1.6 us to set out, 103 us before.
+// out[c] = max(out[c], max_r |x[r, c]|).  HBM-bound: the rows are cut over blockIdx.y so that the
+// pass fills the chip (one block per 128 columns alone was 24 blocks at 3072 channels, each a
+// serial walk of the rows).  kMerge: out set by absmax_init_kernel; block maxima are finite or +inf
+// and never negative, so their int bits order as the floats do and an integer atomic merges them.
+// 4608 x 3072 (28 MB): 6.5 us + 1.6 us to set out, 103 us before.  Otherwise one cut holds all the
+// rows (flk_absmax_cols' rule) and its block writes out itself.
+template <bool kMerge>
 __global__ __launch_bounds__(256) void absmax_cols_kernel(const uint16_t* __restrict__ x, int64_t rows,
                                                           int64_t cols, int64_t stride, int64_t rows_per_block,
-                                                          float* __restrict__ out) {
+                                                          int accumulate, float* __restrict__ out) {
   __shared__ float red[16][129];
   const int64_t c0 = (int64_t)blockIdx.x * 128, r0 = blockIdx.y * rows_per_block;
   const float v = column_absmax<false>(red, x, stride, r0, min(rows, r0 + rows_per_block), cols, c0, nullptr);
   const int64_t c = c0 + threadIdx.x;
-  if (threadIdx.x < 128 && c < cols && v > 0.0f) atomicMax(reinterpret_cast<int*>(out) + c, __float_as_int(v));
+  if (threadIdx.x >= 128 || c >= cols) return;
+  if constexpr (kMerge) {
+    if (v > 0.0f) atomicMax(reinterpret_cast<int*>(out) + c, __float_as_int(v));
+  } else {
+    out[c] = accumulate ? fmaxf(v, out[c]) : v;
+  }
 }
 
 __global__ void smooth_factors_kernel(const float* __restrict__ xa, const float* __restrict__ wa, int64_t k,
@@ -1053,6 +1060,11 @@ int64_t column_rows(int64_t rows, int64_t blocks) {
   return (per + kColRows - 1) / kColRows * kColRows;
 }
 
+// Rows of a column maximum that one block per 128 columns takes in one launch: up to 512 rows are
+// four passes of its loads, less than a second launch costs (us at 3072 columns, cuts and one
+// block: 128 rows 4.2 / 2.6, 256 4.2 / 2.9, 512 4.2 / 3.7; 8 columns 4.6 / 5.4 at 512).
+constexpr int64_t kOneCutRows = 4 * kColRows;
+
 }  // namespace
 
 namespace {
@@ -1096,13 +1108,18 @@ extern "C" int flk_absmax_cols(const void* x, int64_t rows, int64_t cols, int64_
     return FLK_E_ALIGN;
   const int64_t blocks = (cols + 127) / 128;
   if (blocks > INT32_MAX) return FLK_E_INVALID;
-  hipLaunchKernelGGL(absmax_init_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, as_stream(stream), cols,
-                     accumulate, out);
-  if (rows > 0) {
-    const int64_t per = column_rows(rows, blocks);
-    hipLaunchKernelGGL(absmax_cols_kernel, dim3((unsigned)blocks, (unsigned)((rows + per - 1) / per)), dim3(256), 0,
-                       as_stream(stream), static_cast<const uint16_t*>(x), rows, cols, row_stride, per, out);
+  const uint16_t* xp = static_cast<const uint16_t*>(x);
+  const hipStream_t st = as_stream(stream);
+  // Few rows, or blocks that fill the chip without cuts (640 x 131072: two cuts 27.7 us, one 26.3).
+  if (rows <= kOneCutRows || blocks >= 4 * kCUs) {
+    hipLaunchKernelGGL(absmax_cols_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, st, xp, rows, cols, row_stride,
+                       rows, accumulate, out);
+    return flk_launch_status();
   }
+  const int64_t per = column_rows(rows, blocks);
+  hipLaunchKernelGGL(absmax_init_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, st, cols, accumulate, out);
+  hipLaunchKernelGGL(absmax_cols_kernel<true>, dim3((unsigned)blocks, (unsigned)((rows + per - 1) / per)), dim3(256), 0,
+                     st, xp, rows, cols, row_stride, per, accumulate, out);
   return flk_launch_status();
 }
 

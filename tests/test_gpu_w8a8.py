@@ -110,7 +110,7 @@ def test_quantize_weight_full_size_bit_exact(device):
     np.testing.assert_array_equal(host(wq_t), wq_want.T)
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 8), (15, 136), (129, 128), (2 * 128 * 16 + 17, 264), (40000, 8)])
+@pytest.mark.parametrize("rows,cols", [(1, 8), (15, 136), (129, 128), (512, 264), (513, 8), (2 * 128 * 16 + 17, 264), (40000, 8)])
 def test_absmax_cols_row_cuts(device, rows, cols):
     """Row counts around the 128 rows of a block's pass and past one cut per block, into a fresh
     output, into a running maximum and into one that holds a NaN and a negative value."""
@@ -125,6 +125,19 @@ def test_absmax_cols_row_cuts(device, rows, cols):
     start[1], start[2] = float("nan"), -4.0
     run = w8a8.absmax_cols(xd, out=start.to(device))
     np.testing.assert_array_equal(host(run), np.maximum(want, np.nan_to_num(start.numpy().clip(min=0.0))))
+
+
+@pytest.mark.parametrize("rows,cols,count", [(1, 3072, 1), (128, 3072, 1), (512, 8, 1), (513, 3072, 2),
+                                             (640, 128 * 1023, 2), (640, 128 * 1024, 1)])
+def test_absmax_cols_launches(device, rows, cols, count):
+    """Few rows, or columns that fill the chip by themselves, are one launch (a second one costs
+    more than the maxima of 512 rows); either side of the line gives the same maxima."""
+    x = torch.randn(rows, cols, device=device).to(torch.bfloat16)
+    out = torch.full((cols,), 2.0, device=device)
+    for run in (None, out):
+        want = x.float().abs().amax(0)
+        assert torch.equal(w8a8.absmax_cols(x, run), want if run is None else want.clamp(min=2.0))
+        assert len(launches(lambda: w8a8.absmax_cols(x, run))) == count
 
 
 @pytest.mark.parametrize("k,n", [(64, 8), (192, 520), (64, 3072), (64, 3080), (4160, 136)])
