@@ -275,17 +275,42 @@ __global__ __launch_bounds__(256) void weight_scale_kernel(const float* __restri
   w_scale[n] = absmax_scale(v);
 }
 
-// Quantises and transposes one tile of 128 rows (k) x 64 channels.  A thread takes 4 consecutive
-// k of 8 channels, so that four codes leave as one 32-bit LDS write and a WqT row piece as 128
-// contiguous bytes; the 33-word pitch spreads the 64 words of a wave's write over the banks.
+// Codes and transposes a tile of 128 rows (k) x 64 channels.  A thread takes 4 consecutive k (raw, of
+// smoothing factors sj) of 8 channels, so that four codes leave as one 32-bit LDS write and a WqT
+// row piece as 128 contiguous bytes; the 33-word pitch spreads the 64 words of a wave's write over
+// the banks.
+typedef uint32_t WeightTile[64][33];
+
+__device__ __forceinline__ void code_weights(WeightTile& tile, const uint4 (&raw)[4], const float (&sj)[4],
+                                             const float (&sc)[8], const float (&rc)[8]) {
+  const int cg = threadIdx.x & 7, rq = threadIdx.x >> 3;
+  float f[4][8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) unpack_bf16x8(raw[i], f[i]);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float v[4] = {f[0][j] * sj[0], f[1][j] * sj[1], f[2][j] * sj[2], f[3][j] * sj[3]};
+    tile[cg * 8 + j][rq] = quantize4(v, sc[j], rc[j]);
+  }
+}
+
+__device__ __forceinline__ void store_weights(const WeightTile& tile, int8_t* __restrict__ wqt, int n0, int64_t k0,
+                                              int K, int N) {
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const int n = (threadIdx.x >> 3) + it * 32, ch = threadIdx.x & 7;
+    if (n0 + n < N && k0 + ch * 16 < K)
+      *reinterpret_cast<uint4*>(wqt + (int64_t)(n0 + n) * K + k0 + ch * 16) =
+          uint4{tile[n][ch * 4], tile[n][ch * 4 + 1], tile[n][ch * 4 + 2], tile[n][ch * 4 + 3]};
+  }
+}
+
 __global__ __launch_bounds__(256) void quantize_weight_kernel(const uint16_t* __restrict__ w, int64_t w_stride,
                                                               const float* __restrict__ s, int K, int N,
                                                               int8_t* __restrict__ wqt,
                                                               const float* __restrict__ w_scale) {
-  __shared__ uint32_t tile[64][33];
-  const int tid = threadIdx.x;
-  const int cg = tid & 7, rq = tid >> 3;
-  const int n0 = blockIdx.x * 64, nc = n0 + cg * 8;
+  __shared__ WeightTile tile;
+  const int n0 = blockIdx.x * 64, nc = n0 + (threadIdx.x & 7) * 8;
   const bool active = nc < N;
   float sc[8], rc[8];
 #pragma unroll
@@ -294,32 +319,82 @@ __global__ __launch_bounds__(256) void quantize_weight_kernel(const uint16_t* __
   for (int j = 0; j < 8; ++j) rc[j] = 1.0f / sc[j];
   // One tile, but for a K past the grid's 65535 tiles.
   for (int64_t k0 = (int64_t)blockIdx.y * 128; k0 < K; k0 += (int64_t)gridDim.y * 128) {
-    const int64_t kr = k0 + rq * 4;
+    const int64_t kr = k0 + (threadIdx.x >> 3) * 4;
     if (active && kr < K) {
       uint4 raw[4];
-      float sj[4], f[4][8];
+      float sj[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         raw[i] = *reinterpret_cast<const uint4*>(w + (kr + i) * w_stride + nc);
         sj[i] = s[kr + i];
       }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) unpack_bf16x8(raw[i], f[i]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float v[4] = {f[0][j] * sj[0], f[1][j] * sj[1], f[2][j] * sj[2], f[3][j] * sj[3]};
-        tile[cg * 8 + j][rq] = quantize4(v, sc[j], rc[j]);
-      }
+      code_weights(tile, raw, sj, sc, rc);
     }
     __syncthreads();
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      const int n = (tid >> 3) + it * 32, ch = tid & 7;
-      if (n0 + n < N && k0 + ch * 16 < K)
-        *reinterpret_cast<uint4*>(wqt + (int64_t)(n0 + n) * K + k0 + ch * 16) =
-            uint4{tile[n][ch * 4], tile[n][ch * 4 + 1], tile[n][ch * 4 + 2], tile[n][ch * 4 + 3]};
-    }
+    store_weights(tile, wqt, n0, k0, K, N);
     __syncthreads();
+  }
+}
+
+// All of a short weight's rows (K <= 128 kTiles) in one launch: a block holds its 64 channels in
+// registers between the maxima and the codes.  Bound by latency: the three launches above take 7 us
+// however small the weight (us, three launches and one, at 3072 channels: k = 64 8.1 / 3.9, 128
+// 8.2 / 4.0, 256 8.4 / 5.5, 384 8.6 / 6.9, 512 8.9 / 8.4; 512 x 27648 19.4 / 12.7).
+template <int kTiles>
+__global__ __launch_bounds__(256) void quantize_weight_short_kernel(const uint16_t* __restrict__ w, int64_t w_stride,
+                                                                    const float* __restrict__ s, int K, int N,
+                                                                    int8_t* __restrict__ wqt,
+                                                                    float* __restrict__ w_scale) {
+  __shared__ WeightTile tile;
+  __shared__ float red[32][65], scale[64];
+  const int cg = threadIdx.x & 7, rq = threadIdx.x >> 3;
+  const int n0 = blockIdx.x * 64, nc = n0 + cg * 8;
+  const bool active = nc < N;
+  uint4 raw[kTiles][4];
+  float sj[kTiles][4];
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int k = t * 128 + rq * 4 + i;
+      const bool in = active && k < K;
+      raw[t][i] = in ? *reinterpret_cast<const uint4*>(w + k * w_stride + nc) : uint4{0, 0, 0, 0};
+      sj[t][i] = in ? s[k] : 0.0f;
+    }
+  float m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float f[8];
+      unpack_bf16x8(raw[t][i], f);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) m[j] = fmaxf(m[j], fabsf(f[j] * sj[t][i]));
+    }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) red[rq][cg * 8 + j] = m[j];
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    float v = 0.0f;
+#pragma unroll
+    for (int g = 0; g < 32; ++g) v = fmaxf(v, red[g][threadIdx.x]);
+    v = absmax_scale(v);
+    scale[threadIdx.x] = v;
+    if (n0 + (int)threadIdx.x < N) w_scale[n0 + threadIdx.x] = v;
+  }
+  __syncthreads();
+  float sc[8], rc[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    sc[j] = scale[cg * 8 + j];
+    rc[j] = 1.0f / sc[j];
+  }
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) {
+    if (t > 0) __syncthreads();
+    code_weights(tile, raw[t], sj[t], sc, rc);
+    __syncthreads();
+    store_weights(tile, wqt, n0, t * 128, K, N);
   }
 }
 
@@ -1147,6 +1222,17 @@ extern "C" int flk_quantize_weight(const void* w, int64_t w_row_stride, const fl
     return FLK_E_ALIGN;
   const hipStream_t hs = as_stream(stream);
   const uint16_t* wp = static_cast<const uint16_t*>(w);
+  const dim3 channels((unsigned)((n + 63) / 64));
+#define FLK_SHORT(T) \
+  hipLaunchKernelGGL(quantize_weight_short_kernel<T>, channels, dim3(256), 0, hs, wp, w_row_stride, s, k, n, wq_t, w_scale)
+  if (k <= 512) {
+    if (k <= 128) FLK_SHORT(1);
+    else if (k <= 256) FLK_SHORT(2);
+    else if (k <= 384) FLK_SHORT(3);
+    else FLK_SHORT(4);
+    return flk_launch_status();
+  }
+#undef FLK_SHORT
   const int64_t col_blocks = ((int64_t)n + 127) / 128;
   const int64_t per = column_rows(k, col_blocks);
   const int cuts = (int)(((int64_t)k + per - 1) / per);

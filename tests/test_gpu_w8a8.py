@@ -158,7 +158,8 @@ def test_quantize_linear_smooth_equals_two_calls(device, k, n):
     assert float(s[3]) == 1.0 and float(s[5]) == 1.0
 
 
-@pytest.mark.parametrize("k,n", [(64, 8), (192, 72), (128, 264), (4096 + 64, 136)])
+@pytest.mark.parametrize("k,n", [(64, 8), (192, 72), (128, 264), (320, 72), (448, 8), (512, 136), (576, 72),
+                                 (4096 + 64, 136)])
 def test_quantize_weight_tile_edges(device, k, n):
     """k of half a 128-row tile and of several cuts, n off the 64- and 128-channel blocks; every
     byte of WqT is written (the launch uses its front as scratch)."""
@@ -170,6 +171,13 @@ def test_quantize_weight_tile_edges(device, k, n):
     wq_t, ws = w8a8.quantize_weight(w.to(device), torch.from_numpy(s).to(device))
     np.testing.assert_array_equal(host(ws), ws_want)
     np.testing.assert_array_equal(host(wq_t), wq_want.T)
+
+
+@pytest.mark.parametrize("k,count", [(64, 1), (512, 1), (576, 3)])
+def test_quantize_weight_launches(device, k, count):
+    """A weight of up to 512 input channels is one launch: three cost more than its work."""
+    w, s = torch.randn(k, 72, device=device).to(torch.bfloat16), torch.ones(k, device=device)
+    assert len(launches(lambda: w8a8.quantize_weight(w, s))) == count
 
 
 @pytest.mark.parametrize("strided", [False, True])
