@@ -43,10 +43,11 @@ class _KernelNodeParams(ctypes.Structure):
                 ("grid", ctypes.c_uint * 3), ("params", ctypes.c_void_p), ("shared", ctypes.c_uint)]
 
 
-def launches(fn) -> list:
-    """The grid (x, y, z) of every kernel that ``fn`` launches, read from a captured graph."""
+def _kernel_nodes(fn) -> list:
+    """(grid, name) of every kernel that ``fn`` launches, read from a captured graph."""
     from flicker_amd import _lib
     hip = _lib.lib()   # its symbols include those of the HIP runtime it is linked to
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
     fn()
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph(keep_graph=True)
@@ -56,11 +57,21 @@ def launches(fn) -> list:
     assert hip.hipGraphGetNodes(raw, None, ctypes.byref(count)) == 0
     nodes = (ctypes.c_void_p * max(1, count.value))()
     assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(count)) == 0
-    grids = []
+    found = []
     for node in nodes[:count.value]:
         kind, p = ctypes.c_int(-1), _KernelNodeParams()
         assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
         if kind.value == 0:   # hipGraphNodeTypeKernel
             assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
-            grids.append(tuple(p.grid))
-    return grids
+            found.append((tuple(p.grid), hip.hipKernelNameRefByPtr(ctypes.c_void_p(p.func), None).decode()))
+    return found
+
+
+def launches(fn) -> list:
+    """The grid (x, y, z) of every kernel that ``fn`` launches."""
+    return [grid for grid, _ in _kernel_nodes(fn)]
+
+
+def kernel_names(fn) -> list:
+    """The (mangled) name of every kernel that ``fn`` launches."""
+    return [name for _, name in _kernel_nodes(fn)]

@@ -13,7 +13,7 @@ from flicker_amd import w8a8, workloads
 from oracle import w8a8 as Q
 from oracle.numerics import bf16_bits, from_bf16_bits
 
-from ._util import launches
+from ._util import kernel_names, launches
 
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
@@ -138,6 +138,17 @@ def test_absmax_cols_launches(device, rows, cols, count):
         want = x.float().abs().amax(0)
         assert torch.equal(w8a8.absmax_cols(x, run), want if run is None else want.clamp(min=2.0))
         assert len(launches(lambda: w8a8.absmax_cols(x, run))) == count
+
+
+@pytest.mark.parametrize("cols,loads", [(8, 1), (512, 1), (520, 2), (1024, 2), (1536, 3), (1544, 4), (2048, 4),
+                                        (2056, 6), (3080, 6)])
+def test_absmax_rows_loads(device, cols, loads):
+    """A lane has no more loads in flight than its row has chunks (short rows paid for six); the
+    maxima are the same with any."""
+    w = torch.randn(9, cols, device=device).to(torch.bfloat16)
+    assert torch.equal(w8a8.absmax_rows(w), w.float().abs().amax(1))
+    (name,) = kernel_names(lambda: w8a8.absmax_rows(w))
+    assert f"absmax_rows_kernelILi{loads}ELb0EE" in name
 
 
 @pytest.mark.parametrize("k,n", [(64, 8), (192, 520), (64, 3072), (64, 3080), (4160, 136)])
