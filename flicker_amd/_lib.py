@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import pathlib
+import warnings
 
 import torch
 
@@ -144,14 +145,21 @@ def run(name: str, tensors, *args) -> None:
 
 class _Native:
     """The functions of the native per-call path (csrc_host/native.cpp), bound at first use: importing
-    this package loads no library, so a build can replace both.  Where the module is not built
-    for this interpreter each function returns None, and every call takes its Python path."""
+    this package loads no library, so a build can replace both.  The native path runs no library
+    that lib() refuses.  Where the module is not built, or not for this interpreter, torch and
+    library, each function returns None, and every call takes its Python path."""
 
     def __getattr__(self, name: str):
+        if name.startswith("_"):
+            raise AttributeError(name)
+        lib()
         try:
             from . import _native
             fn = getattr(_native, name)
-        except ImportError:
+        except ImportError as error:
+            if any(LIB_PATH.parent.glob("_native*.so")):
+                warnings.warn(f"flicker_amd's native call path is not used, rebuild it: {error}", RuntimeWarning)
+
             def fn(*_):
                 return None
         setattr(self, name, fn)

@@ -1,4 +1,4 @@
-"""Build recipe for libflicker_hip.so (hipcc, gfx950 only) and _native.so (g++, host only).
+"""Build recipe for libflicker_hip.so (hipcc, gfx950 only) and the _native module (g++, host only).
 
 Every ``csrc/*.hip`` file is compiled to an object in parallel, then linked into
 ``flicker_amd/libflicker_hip.so`` next to this file, so the library travels with
@@ -8,6 +8,7 @@ the source tree.  Run ``python -m flicker_amd.build`` or ``__graft_entry__.build
 from __future__ import annotations
 
 import concurrent.futures as cf
+import importlib.machinery
 import os
 import pathlib
 import shutil
@@ -20,7 +21,7 @@ CSRC = PKG / "csrc"
 INCLUDE = ROOT / "include"
 BUILD = PKG / "_build"
 LIB = PKG / "libflicker_hip.so"
-NATIVE = PKG / "_native.so"
+NATIVE = PKG / ("_native" + importlib.machinery.EXTENSION_SUFFIXES[0])   # tagged for this interpreter
 ARCH = "gfx950"
 
 # Packed float32 VALU ops are turned off for all device code; -O3 would otherwise form them.
@@ -81,9 +82,11 @@ def build_native(verbose: bool = False) -> pathlib.Path:
     tmp = NATIVE.with_suffix(".so.tmp")
     _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-          f"-I{includes[0]}", *(f"-isystem{p}" for p in includes[1:]), str(PKG / "csrc_host/native.cpp"), "-o",
+          f'-DFLK_TORCH_VERSION="{torch.__version__}"', f"-I{includes[0]}", *(f"-isystem{p}" for p in includes[1:]), str(PKG / "csrc_host/native.cpp"), "-o",
           str(tmp), f"-L{torch_dir / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip",
           f"-L{PKG}", "-l:libflicker_hip.so", "-Wl,-rpath,$ORIGIN"], verbose)
+    for old in PKG.glob("_native*.so"):
+        old.unlink()
     os.replace(tmp, NATIVE)
     return NATIVE
 

@@ -2,8 +2,6 @@
 
 #include "common.h"
 
-#define FLK_ABI_VERSION 1
-
 extern "C" int flk_abi_version(void) { return FLK_ABI_VERSION; }
 
 extern "C" const char* flk_status_string(int status) {

@@ -18,6 +18,8 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <cstring>
+
 #include "flicker_hip.h"
 
 namespace {
@@ -262,4 +264,21 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nu
 
 }  // namespace
 
-extern "C" __attribute__((visibility("default"))) PyObject* PyInit__native() { return PyModule_Create(&module); }
+// An ImportError unless the library has the ABI and torch the version (its C++ ABI is no other's)
+// that this file was compiled against.  The interpreter's is in the file name.
+extern "C" __attribute__((visibility("default"))) PyObject* PyInit__native() {
+  if (flk_abi_version() != FLK_ABI_VERSION)
+    return PyErr_Format(PyExc_ImportError, "_native is built for ABI %d of libflicker_hip.so, which has %d",
+                        FLK_ABI_VERSION, flk_abi_version());
+  PyObject* const torch = PyImport_ImportModule("torch");
+  PyObject* const version = torch ? PyObject_GetAttrString(torch, "__version__") : nullptr;
+  const char* const text = version ? PyUnicode_AsUTF8(version) : nullptr;
+  PyObject* made = nullptr;
+  if (text && strcmp(text, FLK_TORCH_VERSION) == 0)
+    made = PyModule_Create(&module);
+  else if (text)
+    PyErr_Format(PyExc_ImportError, "_native is built for torch %s, not %s", FLK_TORCH_VERSION, text);
+  Py_XDECREF(version);
+  Py_XDECREF(torch);
+  return made;
+}

@@ -35,7 +35,8 @@ extern "C" {
 #define FLK_E_UNSUPPORTED (-3) /* a shape the library has no kernel for        */
 #define FLK_E_SCRATCH (-4)     /* needs more than a fixed scratch buffer holds  */
 
-/* ABI revision of this header (bumped on any signature change). */
+/* ABI revision of this header (bumped on any signature change), and of the loaded library. */
+#define FLK_ABI_VERSION 1
 int flk_abi_version(void);
 
 /* Static, human-readable text for a return code of any entry point. */

@@ -6,6 +6,7 @@ import ctypes
 import math
 import os
 import re
+import shutil
 import subprocess
 import sys
 
@@ -38,6 +39,44 @@ def test_library_exports_every_declared_symbol(lib):
     for name in syms:
         assert hasattr(lib, name), name
     assert lib.flk_abi_version() == _lib.ABI_VERSION
+
+
+def test_native_path_refuses_the_library_that_the_python_path_refuses(monkeypatch):
+    """A library of another ABI is an error at the native path's first call, as at any other."""
+    monkeypatch.setattr(_lib, "_LIB", None)
+    monkeypatch.setattr(_lib, "ABI_VERSION", _lib.ABI_VERSION + 1)
+    with pytest.raises(_lib.HipLibraryMissing):
+        _lib._Native().linear()
+
+
+@pytest.mark.parametrize("other", ["library", "torch", "interpreter"])
+def test_native_module_is_bound_to_what_it_was_built_for(tmp_path, other):
+    """The module imports beside its own library and torch only, and another interpreter does not
+    find it; the caller is warned and its calls take the Python path."""
+    from flicker_amd import build
+    if other == "interpreter":
+        import sysconfig
+        assert build.NATIVE.name.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
+        assert [p.name for p in build.PKG.glob("_native*.so")] == [build.NATIVE.name]
+        return
+    package = tmp_path / "flicker_amd"
+    package.mkdir()
+    for source in [*build.PKG.glob("*.py"), build.NATIVE]:
+        shutil.copy(source, package)
+    if other == "library":   # every entry point, flk_abi_version among them, returns 99
+        stub = "".join(f"int {name}(void) {{ return 99; }}\n" for name in declared_symbols())
+        subprocess.run(["gcc", "-shared", "-fPIC", "-x", "c", "-", "-o", str(package / "libflicker_hip.so")],
+                       input=stub, text=True, check=True)
+        before = "_lib.ABI_VERSION = 99"
+    else:
+        shutil.copy(_lib.LIB_PATH, package)
+        before = "torch.__version__ = '1.0'"
+    code = (f"import warnings, torch\nfrom flicker_amd import _lib\n{before}\n"
+            "with warnings.catch_warnings(record=True) as seen:\n"
+            "    assert _lib.native.linear() is None\n"
+            "assert 'is built for' in str(seen[-1].message), seen\n")
+    proc = subprocess.run([sys.executable, "-c", code], cwd=tmp_path, capture_output=True, text=True)
+    assert proc.returncode == 0, proc.stderr
 
 
 def test_header_is_plain_c():
