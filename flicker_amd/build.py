@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import concurrent.futures as cf
 import importlib.machinery
+import importlib.util
 import os
 import pathlib
 import shutil
@@ -65,28 +66,35 @@ def build(verbose: bool = False, jobs: int | None = None) -> pathlib.Path:
             f.result()
     tmp = LIB.with_suffix(".so.tmp")
     _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)], verbose)
+    for old in PKG.glob("_native*.so"):   # none is left beside a library it was not linked to
+        old.unlink()
     os.replace(tmp, LIB)
     build_native(verbose)
     return LIB
 
 
-def build_native(verbose: bool = False) -> pathlib.Path:
+def build_native(verbose: bool = False) -> pathlib.Path | None:
     """Compile the host-only Python module over libflicker_hip.so (the hot entry points' per-call
-    path) against this interpreter and its torch; returns its path."""
+    path) against this interpreter and its torch; returns its path.  The package works without
+    it, so a host without g++, torch or their headers gets a warning and None."""
     import sysconfig
+    import warnings
 
+    cxx, spec, python = shutil.which("g++"), importlib.util.find_spec("torch"), sysconfig.get_paths()["include"]
+    torch_dir = pathlib.Path(spec.origin).resolve().parent if spec else pathlib.Path()
+    if not (cxx and spec and (torch_dir / "include/torch/csrc/autograd/python_variable.h").exists()
+            and os.path.exists(os.path.join(python, "Python.h"))):
+        warnings.warn("the native call path is not built: it needs g++ and the headers of Python and torch")
+        return None
     import torch
-    torch_dir = pathlib.Path(torch.__file__).resolve().parent
     includes = [INCLUDE, torch_dir / "include", torch_dir / "include/torch/csrc/api/include",
-                pathlib.Path(hipcc()).resolve().parent.parent / "include", sysconfig.get_paths()["include"]]
+                pathlib.Path(hipcc()).resolve().parent.parent / "include", python]
     tmp = NATIVE.with_suffix(".so.tmp")
-    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-          f'-DFLK_TORCH_VERSION="{torch.__version__}"', f"-I{includes[0]}", *(f"-isystem{p}" for p in includes[1:]), str(PKG / "csrc_host/native.cpp"), "-o",
-          str(tmp), f"-L{torch_dir / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip",
-          f"-L{PKG}", "-l:libflicker_hip.so", "-Wl,-rpath,$ORIGIN"], verbose)
-    for old in PKG.glob("_native*.so"):
-        old.unlink()
+          f'-DFLK_TORCH_VERSION="{torch.__version__}"', f"-I{includes[0]}", *(f"-isystem{p}" for p in includes[1:]),
+          str(PKG / "csrc_host/native.cpp"), "-o", str(tmp), f"-L{torch_dir / 'lib'}", "-ltorch_python", "-ltorch_cpu",
+          "-ltorch", "-lc10", "-lc10_hip", f"-L{PKG}", "-l:libflicker_hip.so", "-Wl,-rpath,$ORIGIN"], verbose)
     os.replace(tmp, NATIVE)
     return NATIVE
 

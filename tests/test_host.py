@@ -79,6 +79,33 @@ def test_native_module_is_bound_to_what_it_was_built_for(tmp_path, other):
     assert proc.returncode == 0, proc.stderr
 
 
+@pytest.mark.parametrize("cxx", ["fails", "missing"])
+def test_build_leaves_no_native_module_of_another_library(tmp_path, monkeypatch, cxx):
+    """A host without g++ still builds the library, as the package works without the native module;
+    whether g++ fails or is missing, no module linked to the replaced library stays."""
+    from flicker_amd import build
+
+    def run(cmd, verbose):
+        if "-fvisibility=hidden" in cmd:
+            raise RuntimeError("build step failed")
+        open(cmd[cmd.index("-o") + 1], "w").close()
+
+    monkeypatch.setattr(build, "_run", run)
+    for name, path in (("PKG", ""), ("BUILD", "_build"), ("LIB", build.LIB.name), ("NATIVE", build.NATIVE.name)):
+        monkeypatch.setattr(build, name, tmp_path / path)
+    for old in (build.NATIVE, tmp_path / "_native.so"):
+        old.touch()
+    if cxx == "missing":
+        which = shutil.which
+        monkeypatch.setattr(build.shutil, "which", lambda exe: None if exe == "g++" else which(exe))
+        with pytest.warns(UserWarning, match="native call path is not built"):
+            assert build.build() == tmp_path / build.LIB.name
+    else:
+        with pytest.raises(RuntimeError, match="build step failed"):
+            build.build()
+    assert build.LIB.exists() and not list(tmp_path.glob("_native*.so"))
+
+
 def test_header_is_plain_c():
     """include/flicker_hip.h is the FFI boundary (ctypes here; cgo or a C caller elsewhere): it
     must parse as C99, not only as C++."""
