@@ -13,13 +13,14 @@ import numpy as np
 import pytest
 import torch
 
-from flicker_amd import _lib, kernels
+from flicker_amd import _lib, kernels, modules
 from oracle import path as P
 from tests._util import abs_stats, describe, to_np
 
 pytestmark = pytest.mark.gpu
 D = 128
 MAX_ABS, MEAN_ABS = 2e-2, 2e-3
+SPLIT_KERNELS = ("attend_kernel<true>", "attend_merge_kernel")
 
 
 def prepped_case(batch, heads, length, seed, scale=1.0):
@@ -35,7 +36,7 @@ def prepped_case(batch, heads, length, seed, scale=1.0):
 
 def run_attend(q, k, v, device, splits=None):
     """Launch below kernels.attend's score-tile check, so any L can be tested; splits=None
-    takes flk_attend_plan's choice (the key-split path on small grids)."""
+    takes the planned launch (halves or key split on small grids), 1 one block per query tile."""
     q, k, v = (t.to(device) for t in (q, k, v))
     out = torch.empty_like(q)
     kernels._launch_attend(q.contiguous(), k.contiguous(), v.contiguous(), out, out.stride()[:3], splits)
@@ -58,9 +59,10 @@ def tight_gate(label, got, want):
     (1, 2, 64), (1, 2, 128), (2, 3, 1536), (1, 2, 4352),
     (1, 1, 1), (1, 2, 63), (1, 2, 65), (1, 2, 100), (1, 2, 257),
 ])
-def test_attend_matches_bounded_oracle(device, batch, heads, length):
+@pytest.mark.parametrize("splits", [None, 1])   # the planned launch; one block per query tile
+def test_attend_matches_bounded_oracle(device, batch, heads, length, splits):
     q, k, v = prepped_case(batch, heads, length, seed=length)
-    got = run_attend(q, k, v, device)
+    got = run_attend(q, k, v, device, splits)
     want = P.attend_bounded(to_np(q), to_np(k), to_np(v))
     tight_gate(f"B{batch} H{heads} L{length}", got, want)
 
@@ -155,26 +157,29 @@ def test_attend_random_shapes_every_launch_equals_one_head_at_a_time(device):
     print("launches exercised:", sorted(seen))
 
 
-def test_attend_peaked_logits(device):
+@pytest.mark.parametrize("splits", [None, 1])
+def test_attend_peaked_logits(device, splits):
     """Large norm scales (bound 11.3 * 2.4^2 = 65 < 80): far-from-uniform attention."""
     q, k, v = prepped_case(1, 2, 512, seed=5, scale=2.4)
-    got = run_attend(q, k, v, device)
+    got = run_attend(q, k, v, device, splits)
     want = P.attend_bounded(to_np(q), to_np(k), to_np(v))
     tight_gate("peaked", got, want)
 
 
-def test_attend_uniform_keys_give_mean_of_values(device):
+@pytest.mark.parametrize("splits", [None, 1])
+def test_attend_uniform_keys_give_mean_of_values(device, splits):
     """All keys equal -> every weight is 1/L -> o = mean(v) (rounded to bf16)."""
     q, k, v = prepped_case(1, 2, 256, seed=6)
     k = k[:, :, :1].expand_as(k).contiguous()
-    got = run_attend(q, k, v, device)
+    got = run_attend(q, k, v, device, splits)
     mean_v = to_np(v).astype(np.float64).mean(axis=2, keepdims=True)
     st = abs_stats(got, np.broadcast_to(mean_v, got.shape))
     print(describe("uniform keys", st))
     assert st["max_abs"] <= 2e-3
 
 
-def test_attend_dominant_key_selects_its_value(device):
+@pytest.mark.parametrize("splits", [None, 1])
+def test_attend_dominant_key_selects_its_value(device, splits):
     """One key aligned with the query at logit ~ 60 outweighs 255 others at ~0."""
     length = 256
     q = torch.zeros(1, 1, length, D)
@@ -184,7 +189,7 @@ def test_attend_dominant_key_selects_its_value(device):
     g = torch.Generator().manual_seed(8)
     v = torch.randn(1, 1, length, D, generator=g)
     q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
-    got = run_attend(q, k, v, device)
+    got = run_attend(q, k, v, device, splits)
     want = np.broadcast_to(to_np(v)[:, :, 7:8], got.shape)
     st = abs_stats(got, want)
     print(describe("dominant key", st))
@@ -205,7 +210,6 @@ def test_attend_python_api_errors(device):
 def test_attend_merged_equals_merge_heads_of_attend(device, batch, heads, length):
     """The token-major epilogue (flk_attend_to) writes exactly merge_heads(attend(q, k, v))
     (modules.py:63-65): same kernel, different store address -> bit-identical."""
-    from flicker_amd import modules
     q, k, v = (t.to(device) for t in prepped_case(batch, heads, length, seed=11 + length))
     want = modules.merge_heads(kernels.attend(q, k, v, block=None if length % 128 == 0 else length))
     got = kernels.attend_merged(q, k, v)
@@ -229,7 +233,7 @@ def test_attend_key_split_matches_oracle(device, batch, heads, length, splits):
     plain sums -- the same gate as the one-pass kernel, and within rounding of it."""
     planned, _ = _lib.attend_plan(batch, heads, length)
     if splits is None:
-        assert planned > 1, "the shape is meant to take the split path"
+        assert kernels.attend_kernels(batch, heads, length) == SPLIT_KERNELS, "meant to take the split path"
     q, k, v = prepped_case(batch, heads, length, seed=length + 3)
     got = run_attend(q, k, v, device, splits)
     want = P.attend_bounded(to_np(q), to_np(k), to_np(v))
@@ -263,9 +267,8 @@ def test_attend_key_split_dominant_key_in_last_range(device):
 
 def test_attend_merged_key_split(device):
     """attend_merged on the split path writes exactly merge_heads of the split attend."""
-    from flicker_amd import modules
     q, k, v = (t.to(device) for t in prepped_case(1, 3, 4608, seed=21))
-    assert _lib.attend_plan(1, 3, 4608)[0] > 1
+    assert kernels.attend_kernels(1, 3, 4608) == SPLIT_KERNELS
     want = modules.merge_heads(kernels.attend(q, k, v))
     got = kernels.attend_merged(q, k, v)
     torch.cuda.synchronize()
@@ -280,7 +283,7 @@ def test_attend_key_split_long_sequence_matches_unsplit(device):
     same sums in another f32 order, so at most one bf16 ulp apart on a few elements."""
     length = 16896
     planned, _ = _lib.attend_plan(1, 1, length)
-    assert planned == 3
+    assert planned == 3 and kernels.attend_kernels(1, 1, length) == SPLIT_KERNELS
     q, k, v = prepped_case(1, 1, length, seed=31)
     split = run_attend(q, k, v, device)
     one = run_attend(q, k, v, device, 1)
@@ -303,7 +306,7 @@ def test_attend_key_split_random_small_grids(device):
         label = f"split {planned} B{batch} H{heads} L{length}"
         print(label, flush=True)
         q, k, v = prepped_case(batch, heads, length, seed=700 + trial)
-        got = run_attend(q, k, v, device)
+        got = run_attend(q, k, v, device, planned)   # by itself attend takes the halves launch for some
         one = run_attend(q, k, v, device, 1)
         diff = np.abs(got.astype(np.float64) - one)
         assert np.all(diff <= 2 * np.abs(one) * 2.0 ** -8 + 1e-6), label
@@ -336,12 +339,23 @@ def test_attend_halves_matches_oracle(device, queries, length):
 
 @pytest.mark.parametrize("batch,heads,length", [(1, 24, 768), (1, 24, 640), (2, 6, 1300), (1, 3, 700)])
 def test_attend_takes_halves(device, batch, heads, length):
-    """The automatic choice takes the halves launch, merged and head-major, every head the same."""
+    """The automatic choice takes the halves launch; merged, head-major and one head at a time in
+    blocks of the same size are the same bits, within rounding of the one-pass kernel."""
     assert kernels.attend_kernels(batch, heads, length) == ("attend_halves_kernel",)
     q, k, v = (t.to(device) for t in prepped_case(batch, heads, length, seed=heads + length))
     got = kernels.attend_merged(q, k, v)
     one = kernels.attend_merged(q, k, v, splits=1)
+    major = kernels.attend(q, k, v, block=length)
     torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), modules.merge_heads(major).view(torch.int16))
+    queries = _lib.attend_halves_plan(batch, heads, length)
+    for b in range(batch):
+        for h in range(heads):
+            d = [t[b, h].contiguous() for t in (q, k, v)]
+            o = torch.empty_like(d[0])
+            _lib.run("flk_attend_halves_to", (*d, o), *(t.data_ptr() for t in d), o.data_ptr(), 1, 1, length, D,
+                     length * D, length * D, D, queries, _lib.stream_of(o))
+            assert torch.equal(o.view(torch.int16), major[b, h].view(torch.int16)), (b, h)
     diff = np.abs(to_np(got).astype(np.float64) - to_np(one))
     assert np.all(diff <= 2 * np.abs(to_np(one)) * 2.0 ** -8 + 1e-6)
     assert np.mean(diff > 0) <= 0.01

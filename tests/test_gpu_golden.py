@@ -53,11 +53,12 @@ def test_qk_prep_golden(device, which):
         assert np.mean(diff > 0) <= 0.01
 
 
-def test_attend_golden(device):
+@pytest.mark.parametrize("splits", [None, 1])
+def test_attend_golden(device, splits):
     g = load("attn.npz")
     q, k, v = (bf16_tensor(g[n], device)[None] for n in ("q_pre", "k", "v"))
     o = torch.empty_like(q)
-    kernels._launch_attend(q.contiguous(), k.contiguous(), v.contiguous(), o, o.stride()[:3], None)
+    kernels._launch_attend(q.contiguous(), k.contiguous(), v.contiguous(), o, o.stride()[:3], splits)
     torch.cuda.synchronize()
     want = g["bounded"].astype(np.float64)
     diff = np.abs(to_np(o)[0] - want)

@@ -165,7 +165,8 @@ def test_graph_replay_attend_key_split(device):
     capture (the graph's own pool), and every replay equals the eager split result."""
     from flicker_amd import _lib
     heads, length = 3, 2048
-    assert _lib.attend_plan(1, heads, length)[0] > 1
+    splits, _ = _lib.attend_plan(1, heads, length)
+    assert splits > 1
 
     def qkv_of(seed):
         g = torch.Generator().manual_seed(seed)
@@ -178,11 +179,11 @@ def test_graph_replay_attend_key_split(device):
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
-        kernels.attend(*static, out=static_o)      # warm-up outside the capture
+        kernels.attend(*static, out=static_o, splits=splits)      # warm-up outside the capture
     torch.cuda.current_stream().wait_stream(side)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        kernels.attend(*static, out=static_o)
+        kernels.attend(*static, out=static_o, splits=splits)
     for seed in (11, 12, 13):
         fresh = tuple(t.to(device) for t in qkv_of(seed))
         for dst, src in zip(static, fresh):
@@ -190,6 +191,6 @@ def test_graph_replay_attend_key_split(device):
         graph.replay()
         torch.cuda.synchronize()
         replayed = static_o.clone()
-        eager = kernels.attend(*fresh)                # eager split work between replays
+        eager = kernels.attend(*fresh, splits=splits)                # eager split work between replays
         torch.cuda.synchronize()
         assert torch.equal(replayed, eager), f"replay with input seed {seed} differs from eager"
