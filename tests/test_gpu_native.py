@@ -63,6 +63,8 @@ def test_double_attention(device, monkeypatch, heads, lengths):
 def test_attend_merged(device, monkeypatch, shape):
     g = torch.Generator().manual_seed(shape[2])
     q, k, v = (0.2 * torch.randn(3, *shape, generator=g)).to(torch.bfloat16).to(device)
+    taken = kernels._native.attend_merged(q, k, v)
+    assert (taken is None) == (shape == (1, 3, 4608, D))   # the key split, whose workspace is the Python path's
     f = lambda: kernels.attend_merged(q, k, v)   # noqa: E731
     same(f(), python_path(monkeypatch, f))
     t = v.transpose(1, 2).contiguous().transpose(1, 2)   # not dense
@@ -76,6 +78,7 @@ def test_linear(device, monkeypatch, lead):
     x = torch.randn(*lead, 256, generator=g).to(torch.bfloat16).to(device)
     qw = w8a8.quantize_linear((0.02 * torch.randn(256, 136, generator=g)).to(torch.bfloat16).to(device),
                               x.reshape(-1, 256).abs().amax(0).float())
+    assert kernels._native.linear(x, qw.wq_t, qw.w_scale, qw.inv_smooth) is not None
     f = lambda: w8a8.linear(x, qw)   # noqa: E731
     same(f(), python_path(monkeypatch, f))
 

@@ -110,7 +110,8 @@ def test_quantize_weight_full_size_bit_exact(device):
     np.testing.assert_array_equal(host(wq_t), wq_want.T)
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 8), (15, 136), (129, 128), (512, 264), (513, 8), (2 * 128 * 16 + 17, 264), (40000, 8)])
+@pytest.mark.parametrize("rows,cols", [(1, 8), (15, 136), (129, 128), (512, 264), (513, 8), (2 * 128 * 16 + 17, 264),
+                                       (40000, 8)])
 def test_absmax_cols_row_cuts(device, rows, cols):
     """Row counts around the 128 rows of a block's pass and past one cut per block, into a fresh
     output, into a running maximum and into one that holds a NaN and a negative value."""
@@ -231,9 +232,10 @@ def test_quantize_act_near_ties(device):
 
 
 @pytest.mark.parametrize("m,k,n", [(300, 256, 520), (1, 128, 4), (257, 3072, 260), (512, 128, 1024),
-                                   (4608, 3072, 9216 // 36), (2600, 384, 6000)])
+                                   (4608, 3072, 9216 // 36), (1153, 3072, 9220), (2600, 384, 6000)])
 def test_gemm_tails_bit_exact(device, m, k, n):
-    """Ragged tiles in both output dimensions; full-range int8 operands.  The last case has
+    """Ragged tiles in both output dimensions; full-range int8 operands.  1153 tokens x 9220
+    channels is a long product in 256 x 256 tiles of one round.  The last case has
     11 x 24 = 264 tiles, more than one round of 256 CUs: the rounds order runs 256 of them
     whole and cuts the queries of the rest into 192-token tiles, ragged ones included."""
     rng = np.random.default_rng(m * 7 + n)
@@ -272,7 +274,8 @@ def test_gemm_rounds_order_bit_exact(device, m, n):
     assert_bits_equal(y, Q.rescale(acc_want, a, ws), f"y {m}x{k}x{n}")
 
 
-@pytest.mark.parametrize("m,k,n", [(17, 3072, 9216), (192, 384, 9216), (193, 128, 9216), (383, 640, 9212),
+@pytest.mark.parametrize("m,k,n", [(17, 3072, 9216), (256, 3072, 9216), (512, 3072, 9216), (192, 384, 9216),
+                                   (193, 128, 9216), (383, 640, 9212),
                                    (385, 384, 9216), (895, 256, 9216), (897, 128, 9216), (2048, 384, 4096),
                                    (2049, 256, 4096)])
 def test_gemm_few_tiles_bit_exact(device, m, k, n):
@@ -290,6 +293,21 @@ def test_gemm_few_tiles_bit_exact(device, m, k, n):
     acc_want = Q.int_gemm(xq, wq)
     np.testing.assert_array_equal(host(acc), acc_want)
     assert_bits_equal(y, Q.rescale(acc_want, a, ws), f"y {m}x{k}x{n}")
+
+
+@pytest.mark.parametrize("m,k,n,kernel", [
+    (17, 3072, 9216, "w8a8_gemm_split_kernelILb0ELb0ELb0ELi2ELi4ELi1E"),
+    (256, 3072, 9216, "w8a8_gemm_split_kernelILb0ELb0ELb0ELi4ELi4ELi1E"),
+    (512, 3072, 9216, "w8a8_gemm_split_kernelILb0ELb0ELb0ELi4ELi2ELi2E"),
+    (1153, 3072, 9220, "w8a8_gemm_kernelILb0E"),
+    (1100, 3072, 8200, "w8a8_gemm_kernelILb0E"),
+])
+def test_gemm_launch_of_a_shape(device, m, k, n, kernel):
+    """The tile sizes that the shapes of the tests above are meant to run."""
+    xq, wq = (torch.zeros(r, k, dtype=torch.int8, device=device) for r in (m, n))
+    a, ws = (torch.ones(r, device=device) for r in (m, n))
+    (name,) = kernel_names(lambda: w8a8.gemm(xq, a, wq, ws))
+    assert kernel in name
 
 
 def test_gemm_random_shapes_bit_exact(device):
@@ -316,9 +334,10 @@ def test_gemm_random_shapes_bit_exact(device):
         assert_bits_equal(y, Q.rescale(acc_want, a, ws), f"y {m}x{k}x{n}")
 
 
-def test_gemm_extreme_operands(device):
+@pytest.mark.parametrize("m,n", [(64, 64), (1100, 8200)])   # few tiles; 256 x 256 tiles
+def test_gemm_extreme_operands(device, m, n):
     """All operands at +-127: the largest |acc| the int32 accumulator sees at K = 3072."""
-    m, k, n = 64, 3072, 64
+    k = 3072
     xq = np.full((m, k), 127, np.int8)
     xq[1::2] = -127
     wq = np.full((k, n), 127, np.int8)
@@ -402,6 +421,8 @@ def _fused_case(device, batch, length, heads, k, scale_dtype, gain, seed):
     (5, 67, 2, 128, torch.bfloat16, 128 ** -0.5),       # batch entries wrapping inside every tile
     (2, 2176, 24, 128, torch.float32, 128 ** -0.5),     # rounds order, batch entries wrapping in 192-token tiles
     (3, 1300, 24, 128, torch.bfloat16, 0.5),            # rounds order, ragged last token tile
+    (384, 3, 24, 128, torch.bfloat16, 0.5),             # short sequences in one round of 256-token tiles
+    (1200, 3, 24, 128, torch.float32, 0.5),             # ... and in the rounds order's 256- and 192-token tiles
 ])
 def test_fused_projection_qk_prep_bit_exact(device, batch, length, heads, k, scale_dtype, gain):
     """flk_w8a8_qk_prep == flk_qk_prep(flk_w8a8_gemm(...)) bit for bit: the epilogue applies
@@ -490,7 +511,8 @@ def test_modulated_activation_bit_exact(device, batch, length, k):
     assert torch.equal(xq2, xq) and torch.equal(a2, a_scale)
 
 
-@pytest.mark.parametrize("k", [8, 504, 512, 520, 1024, 1032, 1536, 1544, 2048, 3072, 3080, 4096, 4104, 6144, 6152, 8192])
+@pytest.mark.parametrize("k", [8, 504, 512, 520, 1024, 1032, 1536, 1544, 2048, 3072, 3080, 4096, 4104, 6144, 6152,
+                               8192])
 def test_quantize_act_widths(device, k):
     """Each split of a row over waves and chunks, full and ragged, with a last block that is not
     full; rows of zeros, of values whose scale is subnormal (1 / a overflows) or small, and of
