@@ -186,7 +186,7 @@ def _launch_qk_prep(qkv, q_scale, k_scale, freqs, num_heads: int, out, out_offse
     """qk_prep's launch.  ``qk_f32``: the plain branch of qkv_prep with float32 scales
     (modules.py:78-80, where rms_norm's product and apply_rope's result stay float32): q and
     k come out float32, unrounded and without a query gain (flk_qk_prep_f32); v stays bf16."""
-    if _native is not None and out is None and not qk_f32 and out_offset == 0 and type(freqs) is Freqs:
+    if out is None and not qk_f32 and out_offset == 0 and type(freqs) is Freqs:
         done = _native.qk_prep(qkv, q_scale, k_scale, freqs.cos, freqs.sin, freqs.q_gain, num_heads)
         if done is not None:
             return done
@@ -329,7 +329,7 @@ def attend_merged(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
     kernel: the attention epilogue writes o[b, t, h*D:(h+1)*D] directly, so the transposing
     copy of merge_heads disappears.  q, k, v (B, H, L, D) bf16 -> (B, L, H*D) bf16; ``out`` may
     be a (B, L, H*D) view whose rows are strided (e.g. columns of a wider buffer)."""
-    if _native is not None and out is None and splits is None:
+    if out is None and splits is None:
         done = _native.attend_merged(q, k, v)
         if done is not None:
             return done

@@ -86,7 +86,7 @@ def double_attention(txt_qkv, img_qkv, txt_scales, img_scales, freqs: Freqs | Po
     batch, num_txt, width = txt_qkv.shape
     num_img = img_qkv.shape[1]
     fused = type(freqs) is Freqs and row_tile(num_txt) is not None and row_tile(num_img) is not None
-    if _native is not None and fused:
+    if fused:
         done = _native.double_attention(txt_qkv, *txt_scales, img_qkv, *img_scales, freqs.cos, freqs.sin,
                                         freqs.q_gain, num_heads)
         if done is not None:

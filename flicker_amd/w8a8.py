@@ -235,7 +235,7 @@ def gemm(xq: torch.Tensor, a_scale: torch.Tensor, wq_t: torch.Tensor, w_scale: t
 
 def linear(x: torch.Tensor, qw: QuantizedLinear, *, out: torch.Tensor | None = None) -> torch.Tensor:
     """int8 stand-in for ``linear(x, w)`` (nn.py:13-14): (..., K) bf16 -> (..., N) bf16."""
-    if _native is not None and out is None:
+    if out is None:
         y = _native.linear(x, qw.wq_t, qw.w_scale, qw.inv_smooth)
         if y is not None:
             return y
