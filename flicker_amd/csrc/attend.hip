@@ -644,10 +644,10 @@ __global__ __launch_bounds__(kThreads, 2) void attend_tile192_kernel(
              o_row_stride);
 }
 
-// Halves launch, for grids that leave CUs idle in one round of 192-query tiles: the block's two
-// waves of a SIMD take the same queries (group qg of four) and the two halves of the keys, so a
-// block of 64, 96 or 128 queries keeps both waves of every SIMD busy and its loop is half as
-// long.  A 64-row ring tile holds one 32-key unit of each half, an iteration is one phase; the
+// Halves launch, for grids that leave CUs idle in one round of 192-query tiles: wave w < 4 takes query
+// group w of four and the first half of the keys, wave w + 4 the second half of the keys for group
+// (w + 2) % 4, so a block of 64, 96 or 128 queries keeps both waves of every SIMD busy and its
+// loop is half as long.  A 64-row ring tile holds one 32-key unit of each half, an iteration is one phase; the
 // halves' acc and l add at the end through LDS (no running max: the sums add as they are), each
 // wave finishing 64 of the 128 output columns.  The price is more copies per MFMA, which is why
 // grids that fill the CUs keep the wider tiles.

@@ -153,9 +153,13 @@ __global__ __launch_bounds__(kThreads) void qk_prep_kernel(
                                                   blockIdx.x);
 }
 
-// Both streams of a double block in one launch (tables form, two heads per group): token blocks
-// [0, first_blocks) of the grid's x take p[0], the rest p[1].  The text stream's 64 token blocks
-// alone leave most of the chip idle, and each launch costs the caller its own call.
+// Both streams of a double block in one launch (tables form): token blocks [0, first_blocks) of the
+// grid's x take p[0], the rest p[1].  At 256 pixels the streams are 768 and 384 short blocks (24
+// heads, two a group), each launch bound by its latency.  An odd head count takes one head per
+// group, where a single stream takes three if it can: with the streams together there are blocks
+// enough (us, one and three heads a group: 3 heads, 512 + 256 tokens 3.1 / 4.2, 512 + 4096 6.0 / 8.7;
+// 9 heads, 512 + 16384 45.5 / 46.0; 15 heads, 512 + 4096 22.7 / 21.9; as two launches of three 7.7,
+// 13.5, 51 and 26.8).
 struct PairStream {
   const uint16_t* qkv;
   int64_t batch_stride, row_stride;

@@ -249,10 +249,10 @@ __global__ void smooth_factors_kernel(const float* __restrict__ xa, const float*
 // Weight (offline), three launches.  The first cuts the rows of W over blockIdx.y and writes each
 // cut's column maxima of |Wh| to part (cut, channel); the second takes their maximum -> w_scale;
 // the third quantises.  part is the front of the WqT buffer itself, which the third launch then
-// overwrites: a cut has at least 64 rows, so its 4 bytes per channel fit the K bytes per
-// channel many times over.  HBM-bound; one block per 64 channels walking all the rows twice
-// filled 144 CUs and waited on each row: 3072 x 9216 took 91 us, 30 us now (10.4 + 2.0 + 17.3).
-// One launch with 32 channels of all the rows in registers, W read once, took 37.
+// overwrites: cuts are of 128 rows or more, the last of 64 or more, so their 4 bytes per channel
+// fit the K bytes per channel many times over.  HBM-bound; one block per 64 channels walking all
+// the rows twice filled 144 CUs and waited on each row: 3072 x 9216 took 91 us, 30 us now (10.4 +
+// 2.0 + 17.3).  One launch with 32 channels of all the rows in registers, W read once, took 37.
 __global__ __launch_bounds__(256) void weight_absmax_kernel(const uint16_t* __restrict__ w, int64_t w_stride,
                                                             const float* __restrict__ s, int K, int N,
                                                             int64_t rows_per_block, float* __restrict__ part) {
@@ -396,22 +396,6 @@ __global__ __launch_bounds__(256) void quantize_weight_short_kernel(const uint16
   }
 }
 
-// Activation (per forward): kRowWaves waves per token row, the row held in registers
-// (kChunks x 8 elements per lane), its sums and its absmax reduced across the waves.
-//
-// kModulate: the row is first the block input x and becomes the projection input
-//   X = bf16(bf16((bf16(1 + scale) * bf16(layer_norm(x)))) + shift)      (modules.py:38-40)
-// with layer_norm(x) = bf16((x - mean) * (1 / sqrt(var + 1e-6))) (nn.py:17-21), the mean and
-// the variance each summed in float64 and rounded to float32 once (bf16 inputs make the f64
-// sum of the row exact, so the mean does not depend on the summation order), every other
-// step one f32 operation.  scale / shift are the modulation rows of the token's batch entry;
-// X is optionally stored (bf16) for other consumers of the modulated input.
-//
-// What bounds it is the latency of the chain load -> sum -> sum -> absmax -> codes and the L2
-// reads of the modulation and the factors (8 bytes a channel for 2 of x), then VALU work: every
-// load is issued before the first reduction, reductions cross lanes by DPP, and a code takes
-// five instructions (quantize4).  Two rows per wave, which share those reads, gain only past
-// ~9000 rows (4%) and lose up to 15% below.
 // op over the 64 lanes of a wave: the 16-lane rows by DPP, then the rows by lane shuffles.
 template <typename T, typename Op>
 __device__ __forceinline__ T wave_reduce(T v, Op op) {
@@ -462,6 +446,23 @@ struct QuantGroup {
   int K;
 };
 
+// Activation (per forward): kRowWaves waves per token row, the row held in registers
+// (kChunks x 8 elements per lane), its sums and its absmax reduced across the waves.
+//
+// kModulate: the row is first the block input x and becomes the projection input
+//   X = bf16(bf16((bf16(1 + scale) * bf16(layer_norm(x)))) + shift)      (modules.py:38-40)
+// with layer_norm(x) = bf16((x - mean) * (1 / sqrt(var + 1e-6))) (nn.py:17-21), the mean and
+// the variance each summed in float64 and rounded to float32 once (bf16 inputs make the f64
+// sum of the row exact, so the mean does not depend on the summation order), every other
+// step one f32 operation.  scale / shift are the modulation rows of the token's batch entry;
+// X is optionally stored (bf16) for other consumers of the modulated input.
+//
+// What bounds it is the latency of the chain load -> sum -> sum -> absmax -> codes and the L2
+// reads of the modulation and the factors (8 bytes a channel for 2 of x), then VALU work: every
+// load is issued before the first reduction, reductions cross lanes by DPP, and a code takes
+// five instructions (quantize4).  Two rows per wave, which share those reads, gain only past
+// ~9000 rows (4%) and lose up to 15% below.
+//
 // kFull: the lanes' chunks end with the row (K = 512 kRowWaves kChunks).
 template <int kRowWaves, int kChunks, bool kFull, bool kModulate>
 __global__ __launch_bounds__(256) void quantize_act_kernel(const QuantGroup grp) {
@@ -1439,7 +1440,9 @@ int64_t plan_tiles(GemmGroup& g, bool both, int tm, int tn) {
 //   128 x 128, one per CU, four stages    256 tokens: 34.6 -> 15.1    384 tokens: 34.6 -> 15.5
 //   128 x 128, two per CU, two stages     512 tokens: 34.7 -> 22.6    896 tokens: 39.4 -> 29.3
 // Past that 256 x 256 tiles, with half the stage copies per product, are faster: at 1152 tokens
-// (648 tiles of 128 x 128) 41.7 against 46.2, at 4608 129 against 149.
+// (648 tiles of 128 x 128) 41.7 against 46.2, at 4608 129 against 149.  The lines are in tiles, not
+// sizes: over N = 128 to 27648 and K = 512 to 8192 (165 shapes on the small tiles' side, plain, 44
+// with the qk_prep epilogue) none was slower than in 256 x 256 tiles.
 template <bool kAcc, bool kQk, bool kScaleF32>
 int launch_group(GemmGroup g, bool both, void* stream) {
   if (!both) g.p[1] = g.p[0];

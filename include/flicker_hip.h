@@ -242,7 +242,7 @@ int flk_attend_balanced_plan(int batch, int heads, int length, int* grid, int64_
  * flk_attend_to with blocks of `queries` = 64, 96 or 128 queries whose waves also cut the keys in
  * two, the halves' sums added on chip: for grids that leave CUs idle in one round of 192-query
  * tiles.  The result differs from flk_attend's in float32 summation order only, and depends on
- * the shape alone.  flk_attend_halves_plan gives the choice for a shape: the smallest of the
+ * the shape (for flk_attend_halves_plan's choice the batch included) alone.  flk_attend_halves_plan gives the choice for a shape: the smallest of the
  * three whose blocks fit the CUs in one round, or 0 where another launch is faster.
  */
 int flk_attend_halves_plan(int batch, int heads, int length, int* queries);

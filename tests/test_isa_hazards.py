@@ -6,9 +6,9 @@ compiler cannot see.  The LDS-DMA copies (global_load_lds_dwordx4) are issued fr
     followed by a VMEM instruction that reads that SGPR needs 5 wait states (gfx9 family);
   * an SALU write of M0 followed by an LDS DMA needs 1 (the asm's own s_nop 0 gives it).
 
-The copies' scalar base operands are meant to come from scalar arithmetic on kernel
-arguments; if a change ever makes the compiler produce one with v_readfirstlane right before
-a copy, the copy would read a stale address.  This test compiles each csrc/*.hip to assembly
+The copies' scalar base operands are meant to come from scalar arithmetic on kernel arguments
+or on a wave index read long before; if a change ever makes the compiler produce one with
+v_readfirstlane right before a copy, the copy would read a stale address.  This test compiles each csrc/*.hip to assembly
 (no GPU needed) and fails on any such sequence."""
 
 import os
