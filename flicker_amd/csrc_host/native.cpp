@@ -6,8 +6,8 @@
 // foreign call) on a 6.5 us kernel.  Each function here takes the common case of one entry point
 // -- plain GPU tensors of the current device, already in the layout the kernels read -- checks
 // it, allocates the outputs and launches.  For anything else it returns None before any launch,
-// and the caller's Python path copies, converts or raises as it always did; so does a call whose
-// launch reports an error status.
+// and the caller's Python path copies, converts or raises as it always did; so does a call that the
+// library refuses.  An error of the HIP runtime is raised here, as that path raises it.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -95,6 +95,16 @@ bool stream_from(PyObject* qkv, PyObject* q_scale, PyObject* k_scale, int64_t he
 
 PyObject* none() { Py_RETURN_NONE; }
 
+// A launch's bad status: None for a refused argument (negative), else _lib.check's HipKernelError.  The
+// launch reads the runtime's pending error and so clears it: a second attempt would hide it.
+PyObject* failed(int status, const char* what) {
+  if (status < 0) return none();
+  PyObject* const lib = PyImport_ImportModule("flicker_amd._lib");
+  PyObject* const raised = lib ? PyObject_CallMethod(lib, "check", "is", status, what) : nullptr;
+  Py_XDECREF(lib);
+  return raised;
+}
+
 PyObject* tuple_of(std::initializer_list<at::Tensor> tensors) {
   PyObject* out = PyTuple_New((Py_ssize_t)tensors.size());
   if (!out) return nullptr;
@@ -123,17 +133,18 @@ bool attend_plan(int64_t batch, int64_t heads, int64_t length, int& queries) {
                      flk_attend_balanced_plan(b, h, l, &grid, &bytes, &counters) == FLK_OK && grid == 0);
 }
 
-// Attention of dense (B, H, L, 128) q, k, v merged to (B, L, H 128); undefined after an error status.
-at::Tensor attend(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, int queries, int device) {
+const char* attend_name(int queries) { return queries ? "flk_attend_halves_to" : "flk_attend_to"; }
+
+// Attention of dense (B, H, L, 128) q, k, v merged to (B, L, H 128) -> out, and its launch's status.
+int attend(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, int queries, int device, at::Tensor& out) {
   const int64_t batch = q.size(0), heads = q.size(1), length = q.size(2);
-  at::Tensor out = empty({batch, length, heads * kDim}, at::kBFloat16, device);
+  out = empty({batch, length, heads * kDim}, at::kBFloat16, device);
   const int64_t bs = length * heads * kDim, hs = kDim, rs = heads * kDim;
   const int b = (int)batch, h = (int)heads, l = (int)length;
-  const int st = queries ? flk_attend_halves_to(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, l, kDim,
-                                                bs, hs, rs, queries, stream_of(device))
-                         : flk_attend_to(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, l, kDim, bs,
-                                         hs, rs, stream_of(device));
-  return st == FLK_OK ? out : at::Tensor();
+  return queries ? flk_attend_halves_to(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, l, kDim, bs, hs,
+                                        rs, queries, stream_of(device))
+                 : flk_attend_to(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, l, kDim, bs, hs, rs,
+                                 stream_of(device));
 }
 
 // qk_prep(qkv, q_scale, k_scale, cos, sin, q_gain, num_heads) -> (q, k, v) or None
@@ -161,7 +172,7 @@ PyObject* qk_prep(PyObject*, PyObject* const* a, Py_ssize_t n) {
                      s.q_scale->scalar_type() == at::kFloat, gain, (int)s.batch, (int)s.length, (int)heads, kDim,
                      q.data_ptr(), k.data_ptr(), v.data_ptr(), s.length, 0, stream_of(device));
   }
-  return st == FLK_OK ? tuple_of({q, k, v}) : none();
+  return st == FLK_OK ? tuple_of({q, k, v}) : failed(st, "flk_qk_prep");
   END_HANDLE_TH_ERRORS
 }
 
@@ -177,11 +188,12 @@ PyObject* attend_merged(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int queries = 0;
   if (!k || !v || !attend_plan(q->size(0), q->size(1), q->size(2), queries)) return none();
   at::Tensor out;
+  int st;
   {
     pybind11::gil_scoped_release release;
-    out = attend(*q, *k, *v, queries, device);
+    st = attend(*q, *k, *v, queries, device, out);
   }
-  return out.defined() ? THPVariable_Wrap(out) : none();
+  return st == FLK_OK ? THPVariable_Wrap(out) : failed(st, attend_name(queries));
   END_HANDLE_TH_ERRORS
 }
 
@@ -203,6 +215,8 @@ PyObject* double_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int queries = 0;
   if (!cos || !sin || !attend_plan(t.batch, heads, length, queries)) return none();
   at::Tensor out;
+  int st;
+  const char* what = "flk_qk_prep_pair";
   {
     pybind11::gil_scoped_release release;
     const int64_t shape[4] = {t.batch, heads, length, kDim};
@@ -210,15 +224,18 @@ PyObject* double_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
                      v = empty(shape, at::kBFloat16, device);
     const float *c = cos->data_ptr<float>(), *s = sin->data_ptr<float>();
     const int64_t skip = t.length * kDim;
-    const int st = flk_qk_prep_pair(
+    st = flk_qk_prep_pair(
         t.qkv->data_ptr(), t.qkv->stride(0), t.qkv->stride(1), c, s, t.q_scale->data_ptr(), t.k_scale->data_ptr(),
         (int)t.length, 0, i.qkv->data_ptr(), i.qkv->stride(0), i.qkv->stride(1), c + skip, s + skip,
         i.q_scale->data_ptr(), i.k_scale->data_ptr(), (int)i.length, t.length, kDim,
         t.q_scale->scalar_type() == at::kFloat, gain, (int)t.batch, (int)heads, kDim, q.data_ptr(), k.data_ptr(),
         v.data_ptr(), length, stream_of(device));
-    if (st == FLK_OK) out = attend(q, k, v, queries, device);
+    if (st == FLK_OK) {
+      what = attend_name(queries);
+      st = attend(q, k, v, queries, device, out);
+    }
   }
-  if (!out.defined()) return none();
+  if (st != FLK_OK) return failed(st, what);
   return tuple_of({out.narrow(1, 0, t.length), out.narrow(1, t.length, i.length)});
   END_HANDLE_TH_ERRORS
 }
@@ -239,6 +256,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!ws || !inv) return none();
   at::Tensor y;
   int st;
+  const char* what = "flk_quantize_act";
   {
     pybind11::gil_scoped_release release;
     const at::Tensor xq = empty({m, k}, at::kChar, device), scale = empty({m}, at::kFloat, device);
@@ -248,11 +266,13 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* const stream = stream_of(device);
     st = flk_quantize_act(x->data_ptr(), k, inv->data_ptr<float>(), (int)m, (int)k, xq.data_ptr<int8_t>(),
                           scale.data_ptr<float>(), stream);
-    if (st == FLK_OK)
+    if (st == FLK_OK) {
+      what = "flk_w8a8_gemm";
       st = flk_w8a8_gemm(xq.data_ptr<int8_t>(), w->data_ptr<int8_t>(), scale.data_ptr<float>(), ws->data_ptr<float>(),
                          (int)m, (int)k, (int)cols, y.data_ptr(), cols, nullptr, stream);
+    }
   }
-  return st == FLK_OK ? THPVariable_Wrap(y) : none();
+  return st == FLK_OK ? THPVariable_Wrap(y) : failed(st, what);
   END_HANDLE_TH_ERRORS
 }
 

@@ -4,7 +4,7 @@ same bits for the calls it takes, and every other call left to the Python path's
 import pytest
 import torch
 
-from flicker_amd import kernels, modules, w8a8
+from flicker_amd import _lib, kernels, modules, w8a8
 
 pytestmark = pytest.mark.gpu
 D = 128
@@ -106,3 +106,32 @@ def test_other_operands_are_left_alone(device):
     assert n.qk_prep() is None and n.attend_merged(1, 2, 3) is None and n.linear(qkv, None, None, None) is None
     with pytest.raises((RuntimeError, ValueError)):
         torch.vmap(lambda t: kernels.qk_prep(t, qs, ks, f, 2)[0])(qkv[None])
+
+
+@pytest.mark.parametrize("call", ["qk_prep", "attend_merged", "double_attention", "linear"])
+def test_runtime_errors_are_raised(device, monkeypatch, call):
+    """An error that the HIP runtime holds when a call launches (here one of a refused host call) is
+    that call's HipKernelError, as on the Python path, and not hidden by a second attempt."""
+    qkv, scales = stream(device, 1, 64, 2, torch.bfloat16, 3)
+    q = torch.ones(3, 1, 2, 64, D, dtype=torch.bfloat16, device=device)
+    x = torch.ones(4, 128, dtype=torch.bfloat16, device=device)
+    qw = w8a8.quantize_linear(torch.ones(128, 8, dtype=torch.bfloat16, device=device), torch.ones(128, device=device))
+    f, joint = tables(device, 64), tables(device, 128)
+    run = {"qk_prep": lambda: kernels.qk_prep(qkv, *scales, f, 2),
+           "attend_merged": lambda: kernels.attend_merged(*q),
+           "double_attention": lambda: modules.double_attention(qkv, qkv, scales, scales, joint, 2),
+           "linear": lambda: w8a8.linear(x, qw)}[call]
+
+    def pending():
+        run()
+        torch.cuda.synchronize()
+        assert _lib.lib().hipSetDevice(99) != 0
+        try:
+            with pytest.raises(_lib.HipKernelError) as error:
+                run()
+        finally:
+            _lib.lib().hipGetLastError()
+        run()   # the error is reported once
+        return str(error.value).split("failed")[1]
+
+    assert pending() == python_path(monkeypatch, pending)
