@@ -1320,7 +1320,9 @@ extern "C" int flk_attend_plan(int batch, int heads, int length, int* splits, in
 // the merge 9 us and 60 ns a block.  Measured (us; heads x tokens, halves against the launch it
 // replaces): 24 x 768 15.5 / 20.7, 24 x 1280 26.2 / 31.9, 12 x 1536 22.7 / 28.8, 6 x 2048 23.0 /
 // 26.1, 5 x 4608 55.7 / 62.4, 1 x 1024 13.2 / 18.5; where the split stays: 3 x 4608 44.5 / 43.4,
-// 1 x 4608 40.5 / 26.4, 3 x 8192 109 / 100.  24 x 1536 (288 blocks of 128) keeps 192-query tiles.
+// 1 x 4608 40.5 / 26.4, 3 x 8192 109 / 100.  24 x 1536 (288 blocks of 128) keeps 192-query tiles,
+// and so do 97 to 128 tokens of 129 to 256 heads, a block of 128 queries a head: no more blocks than
+// one tile of 192 a head, and slower (129 x 97 9.9 / 9.1, 256 x 128 11.4 / 10.5).
 extern "C" int flk_attend_halves_plan(int batch, int heads, int length, int* queries) {
   if (batch < 0 || heads < 0 || length < 0 || !queries) return FLK_E_INVALID;
   *queries = 0;
@@ -1329,7 +1331,7 @@ extern "C" int flk_attend_halves_plan(int batch, int heads, int length, int* que
   int tq = 0, ns_per_key = 0;
   if (half_tiles(length, 64) * bh <= kCUs) tq = 64, ns_per_key = 84;
   else if (half_tiles(length, 96) * bh <= kCUs) tq = 96, ns_per_key = 100;
-  else if (half_tiles(length, 128) * bh <= kCUs) tq = 128, ns_per_key = 120;
+  else if (length > 128 && half_tiles(length, 128) * bh <= kCUs) tq = 128, ns_per_key = 120;
   else return FLK_OK;
   int splits = 1;
   int64_t bytes = 0;
