@@ -1316,11 +1316,12 @@ extern "C" int flk_attend_plan(int batch, int heads, int length, int* splits, in
 
 // The halves launch of a shape: the smallest block of 64, 96 or 128 queries that fits the CUs in one
 // round, unless the key split is faster.  Estimates in ns, fitted to measured launches: a halves
-// block takes 8.4 / 10 / 12 a key and 5 us around them, a split range 17 a key, its partials and
-// the merge 9 us and 60 ns a block.  Measured (us; heads x tokens, halves against the launch it
-// replaces): 24 x 768 15.5 / 20.7, 24 x 1280 26.2 / 31.9, 12 x 1536 22.7 / 28.8, 6 x 2048 23.0 /
-// 26.1, 5 x 4608 55.7 / 62.4, 1 x 1024 13.2 / 18.5; where the split stays: 3 x 4608 44.5 / 43.4,
-// 1 x 4608 40.5 / 26.4, 3 x 8192 109 / 100.  24 x 1536 (288 blocks of 128) keeps 192-query tiles,
+// block takes 8.4 / 10 / 12 a key and 5 us around them, a split range 18 a key, its partials and
+// the merge 9.5 us and 50 ns a block: over 268 shapes of 1 to 24 heads that the split could take,
+// both measured, no choice of the halves is more than 1% slower.  Measured (us; heads x tokens,
+// halves against the launch it replaces): 24 x 768 15.5 / 20.7, 24 x 1280 26.2 / 31.9, 12 x 1536
+// 22.7 / 28.8, 6 x 2048 23.0 / 26.1, 5 x 4608 55.7 / 62.4, 1 x 1024 13.2 / 18.5; where the split
+// stays: 3 x 2700 27.5 / 26.7, 3 x 4608 44.5 / 43.4, 1 x 4608 40.5 / 26.4, 3 x 8192 109 / 100.  24 x 1536 (288 blocks of 128) keeps 192-query tiles,
 // and so do 97 to 128 tokens of 129 to 256 heads, a block of 128 queries a head: no more blocks than
 // one tile of 192 a head, and slower (129 x 97 9.9 / 9.1, 256 x 128 11.4 / 10.5).
 extern "C" int flk_attend_halves_plan(int batch, int heads, int length, int* queries) {
@@ -1337,7 +1338,7 @@ extern "C" int flk_attend_halves_plan(int batch, int heads, int length, int* que
   int64_t bytes = 0;
   flk_attend_plan(batch, heads, length, &splits, &bytes);
   const int64_t halves_ns = 5000 + (int64_t)length * ns_per_key / 10;
-  const int64_t split_ns = 9000 + 17 * (int64_t)length / splits + 60 * splits * q_tiles(length) * bh;
+  const int64_t split_ns = 9500 + 18 * (int64_t)length / splits + 50 * splits * q_tiles(length) * bh;
   if (splits == 1 || halves_ns < split_ns) *queries = tq;
   return FLK_OK;
 }

@@ -175,7 +175,8 @@ def test_attend_halves_plan_and_validation(lib):
     cases = {(1, 24, 640): 64, (1, 24, 641): 96, (1, 24, 960): 96, (1, 24, 961): 128, (1, 24, 1280): 128,
              (1, 24, 1281): 0, (1, 24, 4608): 0, (1, 3, 4608): 0, (1, 1, 4608): 0, (1, 5, 4608): 96, (1, 6, 2048): 64,
              (1, 1, 1): 64, (1, 256, 64): 64, (1, 257, 64): 0, (1, 129, 96): 96, (1, 129, 97): 0, (1, 256, 128): 0,
-             (1, 128, 128): 64, (1, 128, 129): 96, (1, 128, 193): 128, (0, 3, 64): 0, (1, 2, 2 ** 31 - 257): 0}
+             (1, 3, 2400): 64, (1, 3, 2700): 0, (1, 3, 3200): 0, (1, 128, 128): 64, (1, 128, 129): 96,
+             (1, 128, 193): 128, (0, 3, 64): 0, (1, 2, 2 ** 31 - 257): 0}
     for shape, want in cases.items():
         assert _lib.attend_halves_plan(*shape) == want, (shape, _lib.attend_halves_plan(*shape))
     f = lib.flk_attend_halves_to
